@@ -196,7 +196,7 @@ tess_status alloc_all(tess_diagram* d) {
             d->redo.alloc(n + 1) == hipSuccess && d->snbr.alloc(arena_capacity(n)) == hipSuccess &&
             d->sarea.alloc(arena_capacity(n)) == hipSuccess && d->foff.alloc(n + 1) == hipSuccess &&
             d->fsums.alloc((n + 1023) / 1024 + 1) == hipSuccess && d->work1.alloc(1) == hipSuccess &&
-            d->summary.alloc(1) == hipSuccess && d->tredo.alloc(n + 1) == hipSuccess &&
+            d->summary.alloc(kSummarySlots) == hipSuccess && d->tredo.alloc(n + 1) == hipSuccess &&
             d->spill.alloc(n + 1) == hipSuccess && d->fpos.alloc(n) == hipSuccess &&
             d->arena_ctr.alloc(kArenaWords) == hipSuccess;
   d->arena_next = d->arena_ctr.p;
@@ -292,7 +292,8 @@ CellArgs base_args(tess_diagram* d, const Table* t) {
   a.arena_cap = d->arena_cap;
   a.status = d->status.p;
   a.stats = d->opts.collect_stats ? d->stats.p : nullptr;
-  a.summary = d->summary.p;
+  a.summary = &d->summary.p->s;
+  a.summary_mask = kSummarySlots - 1;
   return a;
 }
 
@@ -420,7 +421,7 @@ tess_status compute_cells(tess_diagram* d, const Planner* plan) {
     sch.count[pick_vpl(d) >> 1] = n;  // vpl 1, 2, 4 -> slot 0, 1, 2
   }
   (void)hipEventRecord(ev.e[2], s);
-  if ((st = c->hip(hipMemsetAsync(d->summary.p, 0, sizeof(Summary), s), "memset")) != TESS_OK ||
+  if ((st = c->hip(hipMemsetAsync(d->summary.p, 0, kSummarySlots * sizeof(SummarySlot), s), "memset")) != TESS_OK ||
       (st = c->hip(launch_fill_u32(d->redo.p, 1, 0u, s), "fill")) != TESS_OK ||
       (st = c->hip(launch_fill_u32(d->tredo.p, 1, 0u, s), "fill")) != TESS_OK ||
       (st = c->hip(launch_fill_u32(d->spill.p, 1, 0u, s), "fill")) != TESS_OK ||
@@ -510,11 +511,12 @@ tess_status compute_cells(tess_diagram* d, const Planner* plan) {
                    "compact")) != TESS_OK)
     return st;
   (void)hipEventRecord(ev.e[4], s);
-  Summary sm2;
-  if ((st = c->hip(hipMemcpyAsync(&sm2, d->summary.p, sizeof(Summary), hipMemcpyDeviceToHost, s), "summary")) !=
+  SummarySlot slots[kSummarySlots];
+  if ((st = c->hip(hipMemcpyAsync(slots, d->summary.p, sizeof(slots), hipMemcpyDeviceToHost, s), "summary")) !=
           TESS_OK ||
       (st = c->hip(hipStreamSynchronize(s), "compute")) != TESS_OK)
     return st;
+  const Summary sm2 = summary_total(slots);
   d->tim.bin_ms = ev.ms(0, 1);
   d->tim.plan_ms = ev.ms(1, 2);
   d->tim.cells_ms = ev.ms(2, 3);

@@ -86,7 +86,7 @@ struct tess_batch {
     if (hgrid_pin) (void)hipHostFree(hgrid_pin);
   }
   DevBuf<tess_cell_stats> stats;
-  DevBuf<Summary> summary;
+  DevBuf<SummarySlot> summary;  // kSummarySlots, shared by the sets
   DevBuf<CellArgs> args;
   DevBuf<double> tkey;
   DevBuf<int32_t> toff;
@@ -154,7 +154,7 @@ tess_status make_views(tess_batch* b) {
     d->fpos.view(b->fpos.p + p, d->n);
     d->arena_next = b->arena.p;
     d->arena_cap = arena_capacity(b->N);
-    d->summary.view(b->summary.p + s, 1);
+    d->summary.view(b->summary.p, kSummarySlots);
     if (b->opts.collect_stats) d->stats.view(b->stats.p + p, d->n);
     for (int k = 0; k < 3; ++k) {
       d->lo[k] = 0;
@@ -358,7 +358,7 @@ tess_status enqueue_cells(tess_batch* b, const uint32_t* list_base, const uint32
   tess_status st;
   if (launch_fill_u32(b->ctrl.p, 2, 0u, s) != hipSuccess || launch_fill_u32(b->ctrl.p + kCtrlTab, 4, 0u, s) != hipSuccess ||
       launch_fill_u32((uint32_t*)b->arena.p, 2 * kArenaWords, 0u, s) != hipSuccess ||
-      launch_fill_u32((uint32_t*)b->summary.p, b->nsets * (sizeof(Summary) / 4), 0u, s) != hipSuccess)
+      launch_fill_u32((uint32_t*)b->summary.p, kSummarySlots * (sizeof(SummarySlot) / 4), 0u, s) != hipSuccess)
     return c->fail(TESS_E_DEVICE, "fill");
   BatchArgs a;
   std::memset(&a, 0, sizeof(a));
@@ -494,7 +494,7 @@ tess_status batch_compute(tess_batch* b, const tess_model* m) {
     }
     if ((st = c->hip(hipGraphLaunch(b->gcells.exec, s), "cells graph")) != TESS_OK) return st;
   }
-  std::vector<Summary> sm(b->nsets);
+  SummarySlot slots[kSummarySlots];
   if ((st = c->hip(hipMemcpyAsync(&mail->nredo, b->ctrl.p + kCtrlRedo, 4, hipMemcpyDeviceToHost, s), "redo")) !=
           TESS_OK ||
       (st = c->hip(hipMemcpyAsync(&mail->ntab, b->ctrl.p + kCtrlTab, 8, hipMemcpyDeviceToHost, s), "lists")) !=
@@ -526,7 +526,7 @@ tess_status batch_compute(tess_batch* b, const tess_model* m) {
           TESS_OK ||
       (st = c->hip(hipMemcpyAsync(&mail->arena, b->arena.p + (size_t)kArenaStride * (kArenaParts + 1), 8, hipMemcpyDeviceToHost, s),
                    "arena")) != TESS_OK ||
-      (st = c->hip(hipMemcpyAsync(sm.data(), b->summary.p, sizeof(Summary) * b->nsets, hipMemcpyDeviceToHost, s),
+      (st = c->hip(hipMemcpyAsync(slots, b->summary.p, sizeof(slots), hipMemcpyDeviceToHost, s),
                    "summary")) != TESS_OK ||
       (st = c->hip(hipStreamSynchronize(s), "cells")) != TESS_OK)
     return st;
@@ -557,14 +557,10 @@ tess_status batch_compute(tess_batch* b, const tess_model* m) {
   b->tim.fallback_cells = learned ? nredo : 0;
   b->tim.table_reruns = b->table_reruns;
   b->tim.spill_cells = b->spill_cells;
-  uint64_t bad_cells = 0, flops = 0, inc = 0;
-  for (const Summary& x : sm) {
-    bad_cells += x.degenerate;
-    flops += x.flops;
-    inc += x.incident_cuts;
-  }
-  b->tim.incident_cuts = inc;
-  b->tim.flops = flops;
+  const Summary sum = summary_total(slots);
+  const uint64_t bad_cells = sum.degenerate;
+  b->tim.incident_cuts = sum.incident_cuts;
+  b->tim.flops = sum.flops;
   b->total_faces = total;
   b->computed = true;
   if (failed) return c->fail(TESS_E_CAPACITY, std::to_string(failed) + " cells exceeded the spill workspace limit");
@@ -651,7 +647,7 @@ tess_status tess_batch_create(tess_ctx* ctx, size_t nsets, const double* const* 
             b->base_dev.alloc(nsets + 1) == hipSuccess && b->dend_dev.alloc(nsets) == hipSuccess &&
             b->cbase_dev.alloc(nsets + 1) == hipSuccess && b->bbase_dev.alloc(nsets + 1) == hipSuccess &&
             b->cpd_dev.alloc(nsets) == hipSuccess && b->pblk_dev.alloc(nsets + 1) == hipSuccess &&
-            b->summary.alloc(nsets) == hipSuccess && b->args.alloc(nsets) == hipSuccess &&
+            b->summary.alloc(kSummarySlots) == hipSuccess && b->args.alloc(nsets) == hipSuccess &&
             b->ctrl.alloc(kCtrlWords) == hipSuccess && b->fpos.alloc(N) == hipSuccess &&
             b->tredo.alloc(N) == hipSuccess && b->spill.alloc(N) == hipSuccess && b->arena.alloc(kArenaWords) == hipSuccess &&
             hipHostMalloc((void**)&b->mail, sizeof(Mail), hipHostMallocDefault) == hipSuccess &&

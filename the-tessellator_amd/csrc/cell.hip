@@ -209,6 +209,11 @@ __device__ __forceinline__ double box_gap(int b, double vmin, double size, doubl
 
 __device__ __forceinline__ double stop_thr(double r2) { return (4.0 * r2) * (1.0 + 1e-9); }
 
+// This workgroup's summary counters.
+__device__ __forceinline__ Summary* summary_slot(const CellArgs& A) {
+  return &reinterpret_cast<SummarySlot*>(A.summary)[blockIdx.x & A.summary_mask].s;
+}
+
 // nf consecutive face slots of the arena: in the region of this wave's XCD,
 // else in the shared overflow region; ~0 (and the no-room count bumped)
 // when both are full.  Wave-uniform result.
@@ -1408,14 +1413,12 @@ __device__ __forceinline__ uint32_t cell_body(const CellArgs& A, const int gpos,
       A.status[oi] = status;
     }
     if (A.summary) {
+      Summary* sum = summary_slot(A);
       if (!(status & (TESS_CELL_CAPACITY | TESS_CELL_DEGENERATE)) && !table_rerun) {
-        atomicAdd(&A.summary->flops, (unsigned long long)(flops + oflops_all + 1));
-        atomicAdd(&A.summary->candidates, (unsigned long long)streamed);
-        if (ninc) atomicAdd(&A.summary->incident_cuts, (unsigned long long)ninc);
+        atomicAdd(&sum->flops, (unsigned long long)(flops + oflops_all + 1));
+        if (ninc) atomicAdd(&sum->incident_cuts, (unsigned long long)ninc);
       }
-      if (status & TESS_CELL_DEGENERATE) atomicAdd(&A.summary->degenerate, 1u);
-      if (status & TESS_CELL_CAPACITY) atomicAdd(&A.summary->capacity, 1u);
-      if (status & TESS_CELL_TABLE) atomicAdd(&A.summary->table, 1u);
+      if (status & TESS_CELL_DEGENERATE) atomicAdd(&sum->degenerate, 1u);
     }
     if (GEO != 1 && A.stats) {
       tess_cell_stats st;
@@ -1949,12 +1952,12 @@ __device__ void spill_cell(const CellArgs& A, const int gpos, const SpillArgs& P
     }
     A.status[oi] = status;
     if (A.summary) {
+      Summary* sum = summary_slot(A);
       if (wrote) {
-        atomicAdd(&A.summary->flops, (unsigned long long)(flops + oflops + 1));
-        atomicAdd(&A.summary->candidates, (unsigned long long)streamed);
-        if (ninc) atomicAdd(&A.summary->incident_cuts, (unsigned long long)ninc);
+        atomicAdd(&sum->flops, (unsigned long long)(flops + oflops + 1));
+        if (ninc) atomicAdd(&sum->incident_cuts, (unsigned long long)ninc);
       }
-      if (status & TESS_CELL_DEGENERATE) atomicAdd(&A.summary->degenerate, 1u);
+      if (status & TESS_CELL_DEGENERATE) atomicAdd(&sum->degenerate, 1u);
     }
     if (A.stats) {
       tess_cell_stats st;

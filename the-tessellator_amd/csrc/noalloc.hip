@@ -55,6 +55,7 @@ struct NaArena {
   GridDev grid;
   Summary summary;
   CellArgs args;
+  unsigned char reserved[16];
   int32_t toff[kNaTable];
   int32_t snbr[kNaPoints * kNaFaces];
   uint32_t bins[kNaPoints], sorted[kNaPoints], sort_tmp[kNaPoints], status[kNaPoints];
@@ -251,7 +252,7 @@ extern "C" tess_status tess_compute_noalloc(tess_ctx* ctx, const double* dxyz, s
   a.arena_next = arena_next;
   a.arena_cap = (uint64_t)kNaPoints * kNaFaces;  // the whole scratch arena
   a.status = NA(A, status);
-  a.summary = summary;
+  a.summary = summary;  // one slot (mask 0)
   a.redo = redo + 1;
   a.nredo = redo;
   // capacity 64, then the overflows at 256, then the spill kernel

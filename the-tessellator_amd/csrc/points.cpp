@@ -80,12 +80,12 @@ tess_status tess_diagram_cells_at_particles(tess_diagram* d, const double* xyz, 
       p->foff.alloc(m + 1) != hipSuccess || (p->have_stats && p->stats.alloc(m) != hipSuccess) ||
       T.sites.alloc(3 * m) != hipSuccess || T.snbr.alloc(arena_capacity(m)) != hipSuccess ||
       T.sarea.alloc(arena_capacity(m)) != hipSuccess || T.fsums.alloc((m + 1023) / 1024 + 1) != hipSuccess ||
-      T.summary.alloc(1) != hipSuccess || T.redo.alloc(m + 1) != hipSuccess || T.tredo.alloc(m + 1) != hipSuccess ||
+      T.summary.alloc(kSummarySlots) != hipSuccess || T.redo.alloc(m + 1) != hipSuccess || T.tredo.alloc(m + 1) != hipSuccess ||
       T.spill.alloc(m + 1) != hipSuccess || T.fpos.alloc(m) != hipSuccess || T.arena.alloc(kArenaWords) != hipSuccess)
     return c->fail(TESS_E_NOMEM, "device allocation failed");
   Events ev;
   if ((st = c->hip(hipMemcpyAsync(T.sites.p, xyz, 24 * m, hipMemcpyHostToDevice, s), "upload")) != TESS_OK ||
-      (st = c->hip(hipMemsetAsync(T.summary.p, 0, sizeof(Summary), s), "memset")) != TESS_OK ||
+      (st = c->hip(hipMemsetAsync(T.summary.p, 0, kSummarySlots * sizeof(SummarySlot), s), "memset")) != TESS_OK ||
       (st = c->hip(launch_fill_u32(T.redo.p, 1, 0u, s), "fill")) != TESS_OK ||
       (st = c->hip(launch_fill_u32(T.tredo.p, 1, 0u, s), "fill")) != TESS_OK ||
       (st = c->hip(launch_fill_u32(T.spill.p, 1, 0u, s), "fill")) != TESS_OK ||
@@ -129,7 +129,7 @@ tess_status tess_diagram_cells_at_particles(tess_diagram* d, const double* xyz, 
   a.arena_cap = arena_capacity(m);
   a.status = p->status.p;
   a.stats = p->have_stats ? p->stats.p : nullptr;
-  a.summary = T.summary.p;
+  a.summary = &T.summary.p->s;
   const int vpl = pick_vpl(d);
   // capacity overflows below 256 vertices: the rerun list; at 256: the
   // spill kernel's; shell-table exhaustions: their own list
@@ -174,18 +174,19 @@ tess_status tess_diagram_cells_at_particles(tess_diagram* d, const double* xyz, 
     return st;
   if (p->nbr.alloc(p->total) != hipSuccess || p->area.alloc(p->total) != hipSuccess)
     return c->fail(TESS_E_NOMEM, "device allocation failed");
-  Summary sm2;
+  SummarySlot slots[kSummarySlots];
   float ms[2] = {0, 0};
   if ((st = c->hip(launch_compact(p->fcount.p, p->foff.p, (int)m, T.snbr.p, T.sarea.p, p->nbr.p, p->area.p, s,
                                   T.fpos.p),
                    "compact")) != TESS_OK ||
       (st = c->hip(hipEventRecord(ev.e[2], s), "event")) != TESS_OK ||
-      (st = c->hip(hipMemcpyAsync(&sm2, T.summary.p, sizeof(Summary), hipMemcpyDeviceToHost, s), "summary")) !=
+      (st = c->hip(hipMemcpyAsync(slots, T.summary.p, sizeof(slots), hipMemcpyDeviceToHost, s), "summary")) !=
           TESS_OK ||
       (st = c->hip(hipStreamSynchronize(s), "compact")) != TESS_OK ||
       (st = c->hip(hipEventElapsedTime(&ms[0], ev.e[0], ev.e[1]), "event")) != TESS_OK ||
       (st = c->hip(hipEventElapsedTime(&ms[1], ev.e[1], ev.e[2]), "event")) != TESS_OK)
     return st;
+  const Summary sm2 = summary_total(slots);
   p->ms[0] = ms[0];
   p->ms[1] = ms[1];
   p->reruns = vpl < 4 ? nredo : 0;

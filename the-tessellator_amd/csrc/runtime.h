@@ -209,7 +209,7 @@ struct tess_diagram {
   DevBuf<int32_t> snbr, nbr;
   DevBuf<uint64_t> foff, fsums;
   DevBuf<tess_cell_stats> stats;
-  DevBuf<Summary> summary;
+  DevBuf<SummarySlot> summary;  // kSummarySlots
   DevBuf<uint32_t> work1, redo_list, redo_list2;
   // cells that exhausted the shell table / outgrew the largest LDS variant:
   // count at [0], grid positions from [1]
@@ -250,7 +250,7 @@ struct tess_diagram {
     DevBuf<unsigned long long> arena;
     DevBuf<uint32_t> redo, redo_list, tredo, spill, keys, keys_out, iota, order;
     DevBuf<uint8_t> sort_tmp;
-    DevBuf<Summary> summary;
+    DevBuf<SummarySlot> summary;
   } stmp;
   // geometry of every cell (tess_diagram_compute_geometry)
   DevBuf<uint32_t> geo_count;
