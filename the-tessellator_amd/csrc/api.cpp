@@ -189,9 +189,9 @@ tess_status alloc_all(tess_diagram* d) {
             d->delim.alloc(nb + 1) == hipSuccess && d->cursor.alloc(nb) == hipSuccess &&
             d->sorted.alloc(n) == hipSuccess && d->scratch.alloc(n) == hipSuccess &&
             d->sums.alloc((nb + 1023) / 1024 + 1) == hipSuccess && d->big.alloc(nb) == hipSuccess &&
-            d->misc.alloc(4) == hipSuccess && d->sx.alloc(n) == hipSuccess && d->sy.alloc(n) == hipSuccess &&
+            d->misc.alloc(4) == hipSuccess && d->pts.alloc(n) == hipSuccess &&
             (d->opts.point_order != TESS_ORDER_MORTON || d->codes.alloc(n) == hipSuccess) &&
-            d->sz.alloc(n) == hipSuccess && d->volume.alloc(n) == hipSuccess &&
+            d->volume.alloc(n) == hipSuccess &&
             d->fcount.alloc(n) == hipSuccess && d->status.alloc(n) == hipSuccess &&
             d->redo.alloc(n + 1) == hipSuccess && d->snbr.alloc(arena_capacity(n)) == hipSuccess &&
             d->sarea.alloc(arena_capacity(n)) == hipSuccess && d->foff.alloc(n + 1) == hipSuccess &&
@@ -225,7 +225,7 @@ tess_status bin_enqueue(tess_diagram* d, hipStream_t s) {
   if ((st = c->hip(launch_counting_sort(d->x.p, d->y.p, d->z.p, n, d->grid.p, d->nbins, b, s, key), "sort")) !=
       TESS_OK)
     return st;
-  return c->hip(launch_gather(d->sorted.p, n, d->x.p, d->y.p, d->z.p, d->sx.p, d->sy.p, d->sz.p, s), "gather");
+  return c->hip(launch_gather(d->sorted.p, n, d->x.p, d->y.p, d->z.p, d->pts.p, s), "gather");
 }
 
 tess_status bin(tess_diagram* d) {
@@ -266,10 +266,7 @@ CellArgs base_args(tess_diagram* d, const Table* t) {
   CellArgs a;
   std::memset(&a, 0, sizeof(a));
   a.n = (int)d->n;
-  a.spx = d->sx.p;
-  a.spy = d->sy.p;
-  a.spz = d->sz.p;
-  a.sorted = d->sorted.p;
+  a.pts = d->pts.p;
   a.delim = d->delim.p;
   a.grid = d->grid.p;
   a.tkey = t->key.p;

@@ -70,7 +70,8 @@ struct tess_batch {
   std::vector<size_t> n, pbase;                        // points per set, first point
   std::vector<size_t> bbase, cbase, sbase, partbase;  // delim, bins, scan sums, partial bounds
   // combined device arrays
-  DevBuf<double> x, y, z, sx, sy, sz, part, volume, sarea, area;
+  DevBuf<double> x, y, z, part, volume, sarea, area;
+  DevBuf<PointRec> pts;
   DevBuf<GridDev> grid;
   DevBuf<uint32_t> bins, cnt, delim, cursor, sorted, scratch, sums, big, misc, fcount, status, ctrl;
   DevBuf<int32_t> snbr, nbr;
@@ -131,9 +132,7 @@ tess_status make_views(tess_batch* b) {
     d->x.view(b->x.p + p, d->n);
     d->y.view(b->y.p + p, d->n);
     d->z.view(b->z.p + p, d->n);
-    d->sx.view(b->sx.p + p, d->n);
-    d->sy.view(b->sy.p + p, d->n);
-    d->sz.view(b->sz.p + p, d->n);
+    d->pts.view(b->pts.p + p, d->n);
     d->grid.view(b->grid.p + s, 1);
     d->part.view(b->part.p + b->partbase[s], 6 * nparts);
     d->bins.view(b->bins.p + p, d->n);
@@ -212,9 +211,7 @@ tess_status enqueue_binning(tess_batch* b) {
   a.sorted = b->sorted.p;
   a.big = b->big.p;
   a.misc = b->misc.p;
-  a.sx = b->sx.p;
-  a.sy = b->sy.p;
-  a.sz = b->sz.p;
+  a.pts = b->pts.p;
   if ((st = c->hip(launch_seg_binning(a, s), "binning")) != TESS_OK) return st;
   return c->hip(launch_batch_check(b->delim.p, b->dend_dev.p, b->base_dev.p, (int)b->nsets, b->ctrl.p + kCtrlBad, s),
                 "binning check");
@@ -635,7 +632,7 @@ tess_status tess_batch_create(tess_ctx* ctx, size_t nsets, const double* const* 
   if (N > (size_t)UINT32_MAX || B > (size_t)UINT32_MAX) return ctx->fail(TESS_E_INVALID, "batch too large");
   b->N = N;
   bool ok = b->x.alloc(N) == hipSuccess && b->y.alloc(N) == hipSuccess && b->z.alloc(N) == hipSuccess &&
-            b->sx.alloc(N) == hipSuccess && b->sy.alloc(N) == hipSuccess && b->sz.alloc(N) == hipSuccess &&
+            b->pts.alloc(N) == hipSuccess &&
             b->part.alloc(P) == hipSuccess && b->grid.alloc(nsets) == hipSuccess && b->bins.alloc(N) == hipSuccess &&
             b->sorted.alloc(N) == hipSuccess && b->scratch.alloc(N) == hipSuccess && b->cnt.alloc(C) == hipSuccess &&
             b->cursor.alloc(C) == hipSuccess && b->big.alloc(C) == hipSuccess && b->delim.alloc(B) == hipSuccess &&

@@ -12,7 +12,7 @@
 //   k_sort_cells ascending point index inside each cell (stable order, the
 //                canonical form of celery.rs:357-369), or ascending
 //                (Morton code, index) for the internal order
-//   k_gather     positions in grid order (coalesced candidate loads)
+//   k_gather     positions and ids in grid order (coalesced candidate loads)
 //   k_compact    per-cell staged faces -> CSR
 // All passes are HBM-bound streams over the points or the cells.
 #include "launch.h"
@@ -362,13 +362,11 @@ __global__ __launch_bounds__(256) void k_sort_big(const uint32_t* __restrict__ d
 
 __global__ void k_gather(const uint32_t* __restrict__ sorted, int n, const double* __restrict__ x,
                          const double* __restrict__ y, const double* __restrict__ z,
-                         double* __restrict__ sx, double* __restrict__ sy, double* __restrict__ sz) {
+                         PointRec* __restrict__ pts) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
   const uint32_t i = sorted[k];
-  sx[k] = x[i];
-  sy[k] = y[i];
-  sz[k] = z[i];
+  pts[k] = PointRec{x[i], y[i], z[i], i, 0u};
 }
 
 // ---- many sets at once (a batch): the same passes over every set's
@@ -561,10 +559,9 @@ __global__ __launch_bounds__(256) void k_seg_sort_big(SegBinning a) {
 __global__ void k_seg_gather(SegBinning a) {
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= a.n) return;
-  const uint64_t o = a.pbase[set_of(a.pbase, a.nsets, k)] + a.sorted[k];
-  a.sx[k] = a.x[o];
-  a.sy[k] = a.y[o];
-  a.sz[k] = a.z[o];
+  const uint32_t i = a.sorted[k];
+  const uint64_t o = a.pbase[set_of(a.pbase, a.nsets, k)] + i;
+  a.pts[k] = PointRec{a.x[o], a.y[o], a.z[o], i, 0u};
 }
 
 // Exclusive scan of face counts into u64 offsets: block scan in u64.
@@ -745,8 +742,8 @@ hipError_t launch_scan_u32(const uint32_t* in, int m, uint32_t* out, uint32_t* s
 }
 
 hipError_t launch_gather(const uint32_t* sorted, int n, const double* x, const double* y,
-                         const double* z, double* sx, double* sy, double* sz, hipStream_t s) {
-  hipLaunchKernelGGL(k_gather, dim3(blocks(n, 256)), dim3(256), 0, s, sorted, n, x, y, z, sx, sy, sz);
+                         const double* z, PointRec* pts, hipStream_t s) {
+  hipLaunchKernelGGL(k_gather, dim3(blocks(n, 256)), dim3(256), 0, s, sorted, n, x, y, z, pts);
   return hipGetLastError();
 }
 

@@ -800,12 +800,12 @@ __device__ __forceinline__ uint32_t cell_body(const CellArgs& A, const int gpos,
   // a site of the set excludes itself by index (interface.rs:299-305); an
   // outside site (interface.rs:211-232) excludes nothing
   const bool ext = A.ext != nullptr;
-  const uint32_t self = (uint32_t)uni_i((int)(ext ? 0xffffffffu : A.sorted[gpos]));
+  const uint32_t self = (uint32_t)uni_i((int)(ext ? 0xffffffffu : A.pts[gpos].id));
   // the site and the grid are wave-uniform: scalar registers (the grid read
   // through the constant address space), not vector ones
-  const double sx = uni_d(ext ? A.ext[3 * gpos] : A.spx[gpos]);
-  const double sy = uni_d(ext ? A.ext[3 * gpos + 1] : A.spy[gpos]);
-  const double sz = uni_d(ext ? A.ext[3 * gpos + 2] : A.spz[gpos]);
+  const double sx = uni_d(ext ? A.ext[3 * gpos] : A.pts[gpos].x);
+  const double sy = uni_d(ext ? A.ext[3 * gpos + 1] : A.pts[gpos].y);
+  const double sz = uni_d(ext ? A.ext[3 * gpos + 2] : A.pts[gpos].z);
   typedef const __attribute__((address_space(4))) GridDev ConstGrid;
   const GridDev& G = *(const GridDev*)(ConstGrid*)A.grid;
   const int cpd = G.cpd;
@@ -975,11 +975,12 @@ __device__ __forceinline__ uint32_t cell_body(const CellArgs& A, const int gpos,
         double px = 0, py = 0, pz = 0, d2 = 0;
         if (k < consumed) {
           const uint32_t s = S.cs.st.bstart[ek] + (uint32_t)(k - (int)S.cs.st.bpref[ek]);
-          jidx = A.sorted[s];
+          const PointRec pr = A.pts[s];
+          jidx = pr.id;
           valid = (jidx != self) && (A.target_group < 0 || A.groups[jidx] == A.target_group);
-          px = A.spx[s] - sx;
-          py = A.spy[s] - sy;
-          pz = A.spz[s] - sz;
+          px = pr.x - sx;
+          py = pr.y - sy;
+          pz = pr.z - sz;
           d2 = (px * px + py * py) + pz * pz;
         }
         // every position of the window lies in an entry before the stop one
@@ -1772,12 +1773,12 @@ __device__ double spill_r2(const double* R, int ne2, int lane) {
 __device__ void spill_cell(const CellArgs& A, const int gpos, const SpillArgs& P, SpillWs& W, uint64_t item,
                            int lane) {
   const bool ext = A.ext != nullptr;
-  const uint32_t self = (uint32_t)uni_i((int)(ext ? 0xffffffffu : A.sorted[gpos]));
+  const uint32_t self = (uint32_t)uni_i((int)(ext ? 0xffffffffu : A.pts[gpos].id));
   // the site and the grid are wave-uniform: scalar registers (the grid read
   // through the constant address space), not vector ones
-  const double sx = uni_d(ext ? A.ext[3 * gpos] : A.spx[gpos]);
-  const double sy = uni_d(ext ? A.ext[3 * gpos + 1] : A.spy[gpos]);
-  const double sz = uni_d(ext ? A.ext[3 * gpos + 2] : A.spz[gpos]);
+  const double sx = uni_d(ext ? A.ext[3 * gpos] : A.pts[gpos].x);
+  const double sy = uni_d(ext ? A.ext[3 * gpos + 1] : A.pts[gpos].y);
+  const double sz = uni_d(ext ? A.ext[3 * gpos + 2] : A.pts[gpos].z);
   typedef const __attribute__((address_space(4))) GridDev ConstGrid;
   const GridDev& G = *(const GridDev*)(ConstGrid*)A.grid;
   const int cpd = G.cpd;
@@ -1830,11 +1831,12 @@ __device__ void spill_cell(const CellArgs& A, const int gpos, const SpillArgs& P
       double px = 0, py = 0, pz = 0, d2 = 0;
       if (k < cnt) {
         const uint32_t s = bst + (uint32_t)k;
-        jidx = A.sorted[s];
+        const PointRec pr = A.pts[s];
+        jidx = pr.id;
         valid = (jidx != self) && (A.target_group < 0 || A.groups[jidx] == A.target_group);
-        px = A.spx[s] - sx;
-        py = A.spy[s] - sy;
-        pz = A.spz[s] - sz;
+        px = pr.x - sx;
+        py = pr.y - sy;
+        pz = pr.z - sz;
         d2 = (px * px + py * py) + pz * pz;
       }
       double nx = 0, ny = 0, nz = 0, off = 0;

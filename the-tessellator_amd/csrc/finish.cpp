@@ -66,7 +66,7 @@ tess_status finish_cells(tess_diagram* d, const CellArgs& a0, std::vector<uint32
   int rmax = kSpillRmax0, fmax = kSpillFmax0;
   // status of an item's cell: the original index (grid position -> sorted)
   // or the site itself
-  const uint32_t* sorted = a0.ext ? nullptr : a0.sorted;
+  const uint32_t* sorted = a0.ext ? nullptr : d->sorted.p;
   while (!tab.empty() || !spl.empty()) {
     if (!tab.empty()) {
       if (L >= full) return c->fail(TESS_E_DEVICE, "a cell reached past the full shell table");

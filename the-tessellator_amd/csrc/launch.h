@@ -51,7 +51,7 @@ struct SegBinning {
   uint32_t* sorted = nullptr;   // [n]
   uint32_t* big = nullptr;      // [nb]
   uint32_t* misc = nullptr;     // [2]: scan total, large cells
-  double *sx = nullptr, *sy = nullptr, *sz = nullptr;  // [n] positions in grid order
+  PointRec* pts = nullptr;  // [n] points in grid order
 };
 hipError_t launch_seg_binning(const SegBinning& a, hipStream_t s);
 // The same binning without the in-cell ordering: b.sorted lists the n
@@ -63,7 +63,7 @@ hipError_t launch_grid_order(const double* x, const double* y, const double* z, 
 hipError_t launch_scan_u32(const uint32_t* in, int m, uint32_t* out, uint32_t* sums, uint32_t* total,
                            hipStream_t s);
 hipError_t launch_gather(const uint32_t* sorted, int n, const double* x, const double* y,
-                         const double* z, double* sx, double* sy, double* sz, hipStream_t s);
+                         const double* z, PointRec* pts, hipStream_t s);
 hipError_t launch_face_offsets(const uint32_t* fcount, int n, uint64_t* foff, uint64_t* sums,
                                hipStream_t s);
 // cell o's faces are read at snbr[fpos[o]] (fpos null: at o * kFaceStage)

@@ -43,7 +43,12 @@ constexpr int kNaDevices = 64;
 // The scratch layout (one per GPU).
 struct NaArena {
   double x[kNaPoints], y[kNaPoints], z[kNaPoints];
-  double sx[kNaPoints], sy[kNaPoints], sz[kNaPoints];
+  union {
+    struct {  // of the sort only: the gather overwrites them
+      uint32_t bins[kNaPoints], sort_tmp[kNaPoints];
+    } sort;
+    PointRec pts[kNaPoints];
+  };
   double part[6 * kNaParts];
   double tkey[kNaTable];
   double sarea[kNaPoints * kNaFaces];
@@ -55,10 +60,10 @@ struct NaArena {
   GridDev grid;
   Summary summary;
   CellArgs args;
-  unsigned char reserved[16];
+  unsigned char reserved[40];
   int32_t toff[kNaTable];
   int32_t snbr[kNaPoints * kNaFaces];
-  uint32_t bins[kNaPoints], sorted[kNaPoints], sort_tmp[kNaPoints], status[kNaPoints];
+  uint32_t sorted[kNaPoints], status[kNaPoints];
   uint32_t redo[kNaPoints + 1], redo_list[kNaPoints], spill[kNaPoints + 1], ctr[4];
   uint32_t cnt[kNaBins], delim[kNaBins + 1], cursor[kNaBins], big[kNaBins];
   uint32_t sums[kNaBins / 1024 + 2], misc[4];
@@ -101,7 +106,7 @@ template <class T>
 T* field(NaArena* a, size_t offset) {
   return reinterpret_cast<T*>(reinterpret_cast<uintptr_t>(a) + offset);
 }
-#define NA(a, m) field<std::remove_extent_t<decltype(NaArena::m)>>(a, offsetof(NaArena, m))
+#define NA(a, m) field<std::remove_extent_t<decltype(static_cast<NaArena*>(nullptr)->m)>>(a, offsetof(NaArena, m))
 
 }  // namespace
 
@@ -159,19 +164,19 @@ extern "C" tess_status tess_compute_noalloc(tess_ctx* ctx, const double* dxyz, s
   const int ni = (int)n, nbins = (int)(cpd * cpd * cpd);
   const int nparts = (int)std::min<size_t>(kNaParts, (n + 255) / 256);
   double *x = NA(A, x), *y = NA(A, y), *z = NA(A, z);
-  double *sx = NA(A, sx), *sy = NA(A, sy), *sz = NA(A, sz);
+  PointRec* pts = NA(A, pts);
   GridDev* grid = field<GridDev>(A, offsetof(NaArena, grid));
   uint32_t* delim = NA(A, delim);
   tess_status st;
   // binning (celery.rs:81-414)
-  SortBufs b{NA(A, bins), NA(A, cnt), delim, NA(A, cursor), NA(A, sorted), NA(A, sort_tmp), NA(A, sums),
+  SortBufs b{NA(A, sort.bins), NA(A, cnt), delim, NA(A, cursor), NA(A, sorted), NA(A, sort.sort_tmp), NA(A, sums),
              NA(A, big), NA(A, misc)};
   GridDev hg;
   uint32_t binned = 0;
   if ((st = ctx->hip(launch_soa(dxyz, ni, x, y, z, s), "soa")) != TESS_OK ||
       (st = ctx->hip(launch_bounds(x, y, z, ni, (int)cpd, NA(A, part), nparts, grid, s), "bounds")) != TESS_OK ||
       (st = ctx->hip(launch_counting_sort(x, y, z, ni, grid, nbins, b, s), "sort")) != TESS_OK ||
-      (st = ctx->hip(launch_gather(b.sorted, ni, x, y, z, sx, sy, sz, s), "gather")) != TESS_OK ||
+      (st = ctx->hip(launch_gather(b.sorted, ni, x, y, z, pts, s), "gather")) != TESS_OK ||
       (st = ctx->hip(hipMemcpyAsync(&hg, grid, sizeof(GridDev), hipMemcpyDeviceToHost, s), "grid copy")) != TESS_OK ||
       (st = ctx->hip(hipMemcpyAsync(&binned, delim + nbins, 4, hipMemcpyDeviceToHost, s), "grid copy")) != TESS_OK ||
       (st = ctx->hip(hipStreamSynchronize(s), "binning")) != TESS_OK)
@@ -226,10 +231,7 @@ extern "C" tess_status tess_compute_noalloc(tess_ctx* ctx, const double* dxyz, s
   CellArgs a;
   std::memset(&a, 0, sizeof(a));
   a.n = ni;
-  a.spx = sx;
-  a.spy = sy;
-  a.spz = sz;
-  a.sorted = b.sorted;
+  a.pts = pts;
   a.delim = delim;
   a.grid = grid;
   a.tkey = NA(A, tkey);

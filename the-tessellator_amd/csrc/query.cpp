@@ -140,9 +140,7 @@ tess_status query_impl(tess_diagram* d, int kind, const double* xyz, size_t nq, 
   a.order = ordered ? oorder.p : nullptr;
   a.sorted = d->sorted.p;
   a.delim = d->delim.p;
-  a.sx = d->sx.p;
-  a.sy = d->sy.p;
-  a.sz = d->sz.p;
+  a.pts = d->pts.p;
   a.groups = target_group >= 0 ? d->groups.p : nullptr;
   a.target_group = target_group;
   a.q = qd.p;

@@ -114,11 +114,13 @@ __device__ __forceinline__ void emit_points(const QueryArgs& a, uint32_t s0, uin
     uint32_t id = 0;
     bool keep = false;
     if (valid) {
-      id = a.sorted[s];
+      if (MODE != 1) id = a.sorted[s];
       if (MODE == 0) {
         keep = true;
       } else if (MODE == 1) {
-        const double dx = qx - a.sx[s], dy = qy - a.sy[s], dz = qz - a.sz[s];
+        const PointRec pr = a.pts[s];
+        id = pr.id;
+        const double dx = qx - pr.x, dy = qy - pr.y, dz = qz - pr.z;
         keep = (dx * dx + dy * dy) + dz * dz <= r2;
       } else {
         keep = a.groups[id] == a.target_group;

@@ -197,7 +197,7 @@ struct tess_diagram {
   DevBuf<GridDev> grid;
   DevBuf<double> part;
   DevBuf<uint32_t> bins, cnt, delim, cursor, sorted, scratch, sums, big, misc, inv;
-  DevBuf<double> sx, sy, sz;
+  DevBuf<PointRec> pts;    // points in grid order
   DevBuf<uint32_t> codes;  // Morton codes (TESS_ORDER_MORTON)
   GridDev hgrid;
   bool binned = false;

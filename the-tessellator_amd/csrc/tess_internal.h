@@ -88,13 +88,19 @@ constexpr int kMlpBias = kMlpH + kMlpH + kMlpOutPad;
 constexpr int kMlpParams = kMlpWeights + kMlpBias;
 static_assert(kMlpParams == TESS_MLP_PARAMS, "parameter count");
 
+// A point in grid order: position and original index in one 32-byte record,
+// so that a candidate costs one address and two 16-byte loads (four loads at
+// four addresses from separate arrays: 2M clustered cells 74.4 -> 73.0 ms,
+// 1M radius queries of 124 points 4.62 -> 4.23 ms).
+struct alignas(16) PointRec {
+  double x, y, z;
+  uint32_t id, pad;
+};
+
 struct CellArgs {
   int n;                   // points in the set
   uint32_t summary_mask;   // summary slot of workgroup b: b & summary_mask
-  const double* spx;       // positions in grid order
-  const double* spy;
-  const double* spz;
-  const uint32_t* sorted;  // grid order -> original index
+  const PointRec* pts;     // points in grid order
   const uint32_t* delim;   // CSR delimiters, cpd^3 + 1
   const GridDev* grid;
   const double* tkey;      // shell table (canonical order)
@@ -190,7 +196,7 @@ struct QueryArgs {
   GridDev g;
   const uint32_t* sorted;  // grid-ordered point ids [n]
   const uint32_t* delim;   // [cpd^3 + 1]
-  const double *sx, *sy, *sz;  // gathered coordinates (grid order)
+  const PointRec* pts;     // points in grid order
   const int64_t* groups;   // by point id; null: no group filter
   int64_t target_group;
   const double* q;         // query positions, AoS [3 nq]
