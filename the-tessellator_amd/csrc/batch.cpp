@@ -322,7 +322,7 @@ tess_status learned_order(tess_batch* b, const tess_model* m, uint32_t bounds[4]
   tess_status st;
   for (size_t k = 0; k < b->nsets; ++k) {
     tess_diagram* d = b->views[k].get();
-    if ((st = c->hip(launch_features(d->bins.p, d->delim.p, (int)d->cpd, (int)d->n, b->feat.p + b->pbase[k] * kMlpIn,
+    if ((st = c->hip(launch_features(d->sorted.p, d->bins.p, d->delim.p, (int)d->cpd, (int)d->n, b->feat.p + b->pbase[k] * kMlpIn,
                                      s),
                      "features")) != TESS_OK)
       return st;

@@ -156,7 +156,7 @@ hipError_t launch_site_order(const double* xyz, int m, const GridDev* g, uint32_
 
 // mlp.hip: learned search-radius model (bf16 MFMA, fp32 accumulate)
 hipError_t launch_mfma_probe(const uint16_t* A, const uint16_t* B, float* D, hipStream_t s);
-hipError_t launch_features(const uint32_t* bins, const uint32_t* delim, int cpd, int n, uint16_t* feat,
+hipError_t launch_features(const uint32_t* sorted, const uint32_t* bins, const uint32_t* delim, int cpd, int n, uint16_t* feat,
                            hipStream_t s);
 hipError_t launch_mlp_forward(const uint16_t* X, int n, const uint16_t* W, const float* bias, float* out,
                               hipStream_t s);

@@ -65,7 +65,7 @@ tess_status infer(tess_diagram* d, const tess_model* m) {
   if (d->feat.alloc((size_t)n * kMlpIn) != hipSuccess || d->pred.alloc((size_t)n * kMlpOut) != hipSuccess)
     return c->fail(TESS_E_NOMEM, "device allocation failed");
   tess_status st;
-  if ((st = c->hip(launch_features(d->bins.p, d->delim.p, (int)d->cpd, n, d->feat.p, c->stream), "features")) !=
+  if ((st = c->hip(launch_features(d->sorted.p, d->bins.p, d->delim.p, (int)d->cpd, n, d->feat.p, c->stream), "features")) !=
       TESS_OK)
     return st;
   return c->hip(launch_mlp_forward(d->feat.p, n, m->wbf.p, m->bias.p, d->pred.p, c->stream), "mlp forward");
@@ -146,7 +146,7 @@ tess_status tess_model_create(tess_ctx* ctx, uint64_t seed, tess_model** out) {
   m->ctx = ctx;
   if (m->master.alloc(kMlpParams) != hipSuccess || m->m1.alloc(kMlpParams) != hipSuccess ||
       m->m2.alloc(kMlpParams) != hipSuccess || m->bias.alloc(kMlpBias) != hipSuccess ||
-      m->wbf.alloc(kMlpWeights) != hipSuccess) {
+      m->wbf.alloc(2 * kMlpWeights) != hipSuccess) {
     delete m;
     return ctx->fail(TESS_E_NOMEM, "device allocation failed");
   }
@@ -259,7 +259,7 @@ tess_status tess_model_add_samples(tess_model* m, tess_diagram* d) {
       grow(m->T, (at + n) * kMlpOut, at * kMlpOut, s) != hipSuccess || grow(m->V, at + n, at, s) != hipSuccess)
     return c->fail(TESS_E_NOMEM, "device allocation failed");
   tess_status st;
-  if ((st = c->hip(launch_features(d->bins.p, d->delim.p, (int)d->cpd, (int)n, m->X.p + at * kMlpIn, s),
+  if ((st = c->hip(launch_features(d->sorted.p, d->bins.p, d->delim.p, (int)d->cpd, (int)n, m->X.p + at * kMlpIn, s),
                    "features")) != TESS_OK ||
       (st = c->hip(launch_targets(d->stats.p, (int)n, smallest_edge(d), m->T.p + at * kMlpOut, m->V.p + at, s),
                    "targets")) != TESS_OK ||
@@ -304,7 +304,11 @@ tess_status tess_model_train(tess_model* m, int epochs, int batch, float lr, uin
   if (Tn.alloc(2 * S) != hipSuccess || grad.alloc((size_t)slots * kMlpParams) != hipSuccess ||
       loss.alloc((size_t)nbatches * slots) != hipSuccess || idx.alloc(S) != hipSuccess)
     return c->fail(TESS_E_NOMEM, "device allocation failed");
-  if ((st = c->hip(launch_standardise(m->T.p, S, m->norm, Tn.p, s), "standardise")) != TESS_OK) return st;
+  // (the train step leaves the slots' pad entries alone)
+  if ((st = c->hip(launch_fill_u32(reinterpret_cast<uint32_t*>(grad.p), (size_t)slots * kMlpParams, 0u, s), "fill")) !=
+          TESS_OK ||
+      (st = c->hip(launch_standardise(m->T.p, S, m->norm, Tn.p, s), "standardise")) != TESS_OK)
+    return st;
   std::vector<int> perm(S);
   std::vector<float> lh((size_t)nbatches * slots);
   uint64_t rs = seed;
@@ -450,7 +454,7 @@ tess_status tess_diagram_features(tess_diagram* d, uint16_t* x) {
   tess_status st;
   if (!d->binned && (st = bin(d)) != TESS_OK) return st;
   if (d->feat.alloc(d->n * kMlpIn) != hipSuccess) return c->fail(TESS_E_NOMEM, "device allocation failed");
-  if ((st = c->hip(launch_features(d->bins.p, d->delim.p, (int)d->cpd, (int)d->n, d->feat.p, c->stream),
+  if ((st = c->hip(launch_features(d->sorted.p, d->bins.p, d->delim.p, (int)d->cpd, (int)d->n, d->feat.p, c->stream),
                    "features")) != TESS_OK)
     return st;
   return c->hip(hipMemcpy(x, d->feat.p, 2 * d->n * kMlpIn, hipMemcpyDeviceToHost), "download");
@@ -492,6 +496,8 @@ tess_status tess_mlp_gradient(tess_model* m, const uint16_t* x, const float* t, 
   if ((st = c->hip(hipMemcpy(X.p, x, 2 * n * kMlpIn, hipMemcpyHostToDevice), "upload")) != TESS_OK ||
       (st = c->hip(hipMemcpy(T.p, t, 4 * n * kMlpOut, hipMemcpyHostToDevice), "upload")) != TESS_OK ||
       (st = c->hip(hipMemcpy(idx.p, id.data(), 4 * n, hipMemcpyHostToDevice), "upload")) != TESS_OK ||
+      (st = c->hip(launch_fill_u32(reinterpret_cast<uint32_t*>(G.p), (size_t)slots * kMlpParams, 0u, s), "fill")) !=
+          TESS_OK ||
       (st = c->hip(launch_mlp_train_step(X.p, T.p, idx.p, (int)n, 1.f / (float)n, m->wbf.p, m->bias.p, G.p, L.p, s),
                    "train step")) != TESS_OK ||
       (st = c->hip(launch_grad_sum(G.p, slots, Gs.p, s), "grad sum")) != TESS_OK)
