@@ -166,6 +166,18 @@ hipError_t launch_mlp_train_step(const uint16_t* X, const float* T, const int* i
 hipError_t launch_targets(const tess_cell_stats* st, int n, double smin, float* T, uint16_t* vmax, hipStream_t s);
 hipError_t launch_grad_sum(const float* grad, int nslots, float* out, hipStream_t s);
 hipError_t launch_standardise(const float* T, size_t n, const float norm[4], float* Tn, hipStream_t s);
+// Predictions in length units and candidates: exp(norm[1] y0 + norm[0]) smin
+// and expm1(norm[3] y1 + norm[2]).
+struct PredictScale {
+  float norm[4];
+  double smin;
+};
+hipError_t launch_predictions(const float* y, int n, const PredictScale& p, float* out, hipStream_t s);
+// Routing calibration: bins of a quarter in log(1 + C), [0, 20); hist holds 3
+// kCalibBins zeros: all samples, those past 64 vertices, those past 128.
+constexpr int kCalibBins = 80;
+hipError_t launch_calibration(const float* y, const uint16_t* vmax, size_t n, float scale, float shift,
+                              uint32_t* hist, hipStream_t s);
 hipError_t launch_weights_from_master(const float* master, uint16_t* wbf, float* bias, hipStream_t s);
 hipError_t launch_adam(const float* grad, int nslots, float* master, float* m1, float* m2, uint16_t* wbf,
                        float* bias, float lr, float b1c, float b2c, hipStream_t s);

@@ -344,35 +344,28 @@ tess_status tess_model_train(tess_model* m, int epochs, int batch, float lr, uin
   // so the cells routed to the larger capacity are those whose bins mostly
   // need it.  No bin at or above one in five: the route stays closed.
   DevBuf<float> Y;
-  if (Y.alloc(2 * S) != hipSuccess) return c->fail(TESS_E_NOMEM, "device allocation failed");
-  std::vector<float> y(2 * S);
-  std::vector<uint16_t> V(S);
+  DevBuf<uint32_t> hist;
+  uint32_t counts[3 * kCalibBins];
+  if (Y.alloc(2 * S) != hipSuccess || hist.alloc(3 * kCalibBins) != hipSuccess)
+    return c->fail(TESS_E_NOMEM, "device allocation failed");
   if ((st = c->hip(launch_mlp_forward(m->X.p, (int)S, m->wbf.p, m->bias.p, Y.p, s), "mlp forward")) != TESS_OK ||
-      (st = c->hip(hipMemcpyAsync(y.data(), Y.p, 4 * y.size(), hipMemcpyDeviceToHost, s), "download")) != TESS_OK ||
-      (st = c->hip(hipMemcpyAsync(V.data(), m->V.p, 2 * S, hipMemcpyDeviceToHost, s), "download")) != TESS_OK ||
+      (st = c->hip(launch_fill_u32(hist.p, 3 * kCalibBins, 0u, s), "fill")) != TESS_OK ||
+      (st = c->hip(launch_calibration(Y.p, m->V.p, S, m->norm[3], m->norm[2], hist.p, s), "calibrate")) != TESS_OK ||
+      (st = c->hip(hipMemcpyAsync(counts, hist.p, sizeof(counts), hipMemcpyDeviceToHost, s), "download")) != TESS_OK ||
       (st = c->hip(hipStreamSynchronize(s), "calibrate")) != TESS_OK)
     return st;
-  constexpr int kBins = 80;  // log(1 + C) in [0, 20)
-  const int caps[2] = {64, 128};
   for (int r = 0; r < 2; ++r) {
-    std::vector<uint64_t> cnt(kBins, 0), over(kBins, 0);
+    const uint32_t* cnt = counts;
+    const uint32_t* over = counts + (1 + r) * kCalibBins;
     bool any = false;
-    for (size_t i = 0; i < S; ++i) {
-      const float v = y[2 * i + 1] * m->norm[3] + m->norm[2];
-      const int bin = std::min(kBins - 1, std::max(0, (int)std::floor(v * 4.0f)));
-      cnt[bin]++;
-      if (V[i] > caps[r]) {
-        over[bin]++;
-        any = true;
-      }
-    }
+    for (int bin = 0; bin < kCalibBins; ++bin) any = any || over[bin];
     float t = std::numeric_limits<float>::infinity();
     if (any) {
       int hi = -1;  // highest populated bin below one in five
       bool high_seen = false;
-      for (int bin = 0; bin < kBins; ++bin) {
+      for (int bin = 0; bin < kCalibBins; ++bin) {
         if (cnt[bin] < 20) continue;
-        if (5 * over[bin] < cnt[bin])
+        if (5ull * over[bin] < cnt[bin])
           hi = bin;
         else
           high_seen = true;
@@ -394,17 +387,16 @@ tess_status tess_diagram_predict(tess_diagram* d, const tess_model* m, float* ou
   tess_status st;
   if (!d->binned && (st = bin(d)) != TESS_OK) return st;
   if ((st = infer(d, m)) != TESS_OK) return st;
-  std::vector<float> y(2 * d->n);
-  if ((st = c->hip(hipMemcpyAsync(y.data(), d->pred.p, 4 * y.size(), hipMemcpyDeviceToHost, c->stream),
-                   "download")) != TESS_OK ||
+  // (the raw outputs stay in d->pred for the schedule's use of them)
+  DevBuf<float> res;
+  if (res.alloc(2 * d->n) != hipSuccess) return c->fail(TESS_E_NOMEM, "device allocation failed");
+  PredictScale p;
+  std::memcpy(p.norm, m->norm, sizeof(p.norm));
+  p.smin = smallest_edge(d);
+  if ((st = c->hip(launch_predictions(d->pred.p, (int)d->n, p, res.p, c->stream), "predict")) != TESS_OK ||
       (st = c->hip(hipStreamSynchronize(c->stream), "predict")) != TESS_OK)
     return st;
-  const double smin = smallest_edge(d);
-  for (size_t i = 0; i < d->n; ++i) {
-    out[2 * i] = (float)(std::exp((double)y[2 * i] * m->norm[1] + m->norm[0]) * smin);
-    out[2 * i + 1] = (float)std::expm1((double)y[2 * i + 1] * m->norm[3] + m->norm[2]);
-  }
-  return TESS_OK;
+  return c->hip(download(c, out, res.p, 8 * d->n), "download");
 }
 
 tess_status tess_diagram_compute_learned(tess_diagram* d, const tess_model* m) {
