@@ -186,7 +186,7 @@ tess_status alloc_all(tess_diagram* d) {
   bool ok = d->x.alloc(n) == hipSuccess && d->y.alloc(n) == hipSuccess && d->z.alloc(n) == hipSuccess &&
             d->grid.alloc(1) == hipSuccess && d->part.alloc(6 * (size_t)nparts) == hipSuccess &&
             d->bins.alloc(n) == hipSuccess && d->cnt.alloc(nb) == hipSuccess &&
-            d->delim.alloc(nb + 1) == hipSuccess && d->cursor.alloc(nb) == hipSuccess &&
+            d->delim.alloc(nb + 1) == hipSuccess && 
             d->sorted.alloc(n) == hipSuccess && d->scratch.alloc(n) == hipSuccess &&
             d->sums.alloc((nb + 1023) / 1024 + 1) == hipSuccess && d->big.alloc(nb) == hipSuccess &&
             d->misc.alloc(4) == hipSuccess && d->pts.alloc(n) == hipSuccess &&
@@ -214,7 +214,7 @@ tess_status bin_enqueue(tess_diagram* d, hipStream_t s) {
   if ((st = c->hip(launch_bounds(d->x.p, d->y.p, d->z.p, n, (int)d->cpd, d->part.p, nparts, d->grid.p, s),
                    "bounds")) != TESS_OK)
     return st;
-  SortBufs b{d->bins.p, d->cnt.p, d->delim.p, d->cursor.p, d->sorted.p, d->scratch.p, d->sums.p, d->big.p,
+  SortBufs b{d->bins.p, d->cnt.p, d->delim.p, d->sorted.p, d->scratch.p, d->sums.p, d->big.p,
              d->misc.p};
   const uint32_t* key = nullptr;
   if (d->opts.point_order == TESS_ORDER_MORTON) {  // a cell's points in the internal (Morton) order
@@ -225,6 +225,11 @@ tess_status bin_enqueue(tess_diagram* d, hipStream_t s) {
   if ((st = c->hip(launch_counting_sort(d->x.p, d->y.p, d->z.p, n, d->grid.p, d->nbins, b, s, key), "sort")) !=
       TESS_OK)
     return st;
+  if (d->have_groups) {
+    if (d->sgroups.alloc(d->n) != hipSuccess) return c->fail(TESS_E_NOMEM, "device allocation failed");
+    if ((st = c->hip(launch_gather_groups(d->sorted.p, n, d->groups.p, d->sgroups.p, s), "gather")) != TESS_OK)
+      return st;
+  }
   return c->hip(launch_gather(d->sorted.p, n, d->x.p, d->y.p, d->z.p, d->pts.p, s), "gather");
 }
 
@@ -277,7 +282,7 @@ CellArgs base_args(tess_diagram* d, const Table* t) {
     a.lo[k] = d->lo[k];
     a.hi[k] = d->hi[k];
   }
-  a.groups = d->have_groups ? d->groups.p : nullptr;
+  a.groups = d->have_groups ? d->sgroups.p : nullptr;
   a.target_group = -1;
   a.radius_limit = std::numeric_limits<double>::quiet_NaN();
   a.volume = d->volume.p;

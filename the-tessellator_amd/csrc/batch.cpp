@@ -139,7 +139,6 @@ tess_status make_views(tess_batch* b) {
     d->sorted.view(b->sorted.p + p, d->n);
     d->scratch.view(b->scratch.p + p, d->n);
     d->cnt.view(b->cnt.p + b->cbase[s], nb);
-    d->cursor.view(b->cursor.p + b->cbase[s], nb);
     d->big.view(b->big.p + b->cbase[s], nb);
     d->delim.view(b->delim.p + b->bbase[s], nb + 1);
     d->sums.view(b->sums.p + b->sbase[s], (nb + 1023) / 1024 + 1);

@@ -1211,7 +1211,7 @@ __device__ __forceinline__ uint32_t cell_body(const CellArgs& args, const int gp
           const uint32_t s = S.cs.st.bstart[ek] + (uint32_t)(k - (int)S.cs.st.bpref[ek]);
           const PointRec pr = B.pts[s];
           jidx = pr.id;
-          valid = (jidx != self) && (skip_cells || B.groups[jidx] == B.target_group);
+          valid = (jidx != self) && (skip_cells || B.groups[s] == B.target_group);
           px = pr.x - sx;
           py = pr.y - sy;
           pz = pr.z - sz;
@@ -2088,7 +2088,7 @@ __device__ void spill_cell(const CellArgs& A, const int gpos, const SpillArgs& P
         const uint32_t s = bst + (uint32_t)k;
         const PointRec pr = A.pts[s];
         jidx = pr.id;
-        valid = (jidx != self) && (A.target_group < 0 || A.groups[jidx] == A.target_group);
+        valid = (jidx != self) && (A.target_group < 0 || A.groups[s] == A.target_group);
         px = pr.x - sx;
         py = pr.y - sy;
         pz = pr.z - sz;

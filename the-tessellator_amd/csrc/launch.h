@@ -8,12 +8,11 @@ namespace tess {
 hipError_t launch_soa(const double* xyz, int n, double* x, double* y, double* z, hipStream_t s);
 hipError_t launch_bounds(const double* x, const double* y, const double* z, int n, int cpd,
                          double* part, int nparts, GridDev* g, hipStream_t s);
-// counting sort: bins/cnt/delim/cursor/sorted/scratch sized by the caller
+// counting sort: bins/cnt/delim/sorted/scratch sized by the caller
 struct SortBufs {
   uint32_t* bins;     // [n]
   uint32_t* cnt;      // [nbins]
   uint32_t* delim;    // [nbins + 1]
-  uint32_t* cursor;   // [nbins] (grid-order binning only)
   uint32_t* sorted;   // [n]
   uint32_t* scratch;  // [n]: slots in the cell ranges, then the in-cell sort's copy
   uint32_t* sums;     // [ceil(nbins / 1024) + 1]
@@ -56,12 +55,13 @@ struct SegBinning {
 hipError_t launch_seg_binning(const SegBinning& a, hipStream_t s);
 // The same binning without the in-cell ordering: b.sorted lists the n
 // positions grid cell by grid cell, in no set order inside a cell (only
-// bins, cnt, delim, cursor, sorted, sums and misc are used)
+// bins, cnt, delim, sorted, scratch, sums and misc are used)
 hipError_t launch_grid_order(const double* x, const double* y, const double* z, int n, const GridDev* g,
                              int nbins, const SortBufs& b, hipStream_t s);
 // exclusive scan of m u32 (sums: ceil(m / 1024) + 1 entries); *total = sum
 hipError_t launch_scan_u32(const uint32_t* in, int m, uint32_t* out, uint32_t* sums, uint32_t* total,
                            hipStream_t s);
+hipError_t launch_gather_groups(const uint32_t* sorted, int n, const int64_t* groups, int64_t* out, hipStream_t s);
 hipError_t launch_gather(const uint32_t* sorted, int n, const double* x, const double* y,
                          const double* z, PointRec* pts, hipStream_t s);
 hipError_t launch_face_offsets(const uint32_t* fcount, int n, uint64_t* foff, uint64_t* sums,

@@ -60,12 +60,12 @@ struct NaArena {
   GridDev grid;
   Summary summary;
   CellArgs args;
-  unsigned char reserved[40];
+  unsigned char reserved[40 + 4 * kNaBins];
   int32_t toff[kNaTable];
   int32_t snbr[kNaPoints * kNaFaces];
   uint32_t sorted[kNaPoints], status[kNaPoints];
   uint32_t redo[kNaPoints + 1], redo_list[kNaPoints], spill[kNaPoints + 1], ctr[4];
-  uint32_t cnt[kNaBins], delim[kNaBins + 1], cursor[kNaBins], big[kNaBins];
+  uint32_t cnt[kNaBins], delim[kNaBins + 1], big[kNaBins];
   uint32_t sums[kNaBins / 1024 + 2], misc[4];
   uint32_t spill_u[kNaSpillBlocks * (2 * (kNaFmax + 1) + 7 * kNaFmax)];
   uint8_t spill_b[kNaSpillBlocks * (kNaRmax + kNaFmax)];
@@ -169,7 +169,7 @@ extern "C" tess_status tess_compute_noalloc(tess_ctx* ctx, const double* dxyz, s
   uint32_t* delim = NA(A, delim);
   tess_status st;
   // binning (celery.rs:81-414)
-  SortBufs b{NA(A, sort.bins), NA(A, cnt), delim, NA(A, cursor), NA(A, sorted), NA(A, sort.sort_tmp), NA(A, sums),
+  SortBufs b{NA(A, sort.bins), NA(A, cnt), delim, NA(A, sorted), NA(A, sort.sort_tmp), NA(A, sums),
              NA(A, big), NA(A, misc)};
   GridDev hg;
   uint32_t binned = 0;

@@ -119,17 +119,17 @@ tess_status query_impl(tess_diagram* d, int kind, const double* xyz, size_t nq, 
   // Large sets: take the queries in grid order of their positions (the
   // results do not depend on the order the wavefronts take them in).
   DevBuf<double>&ox = T.ox, &oy = T.oy, &oz = T.oz;
-  DevBuf<uint32_t>&obins = T.obins, &ocnt = T.ocnt, &odelim = T.odelim, &ocursor = T.ocursor, &oorder = T.oorder,
+  DevBuf<uint32_t>&obins = T.obins, &ocnt = T.ocnt, &odelim = T.odelim, &orank = T.orank, &oorder = T.oorder,
                    &osums = T.osums, &omisc = T.omisc;
   const bool ordered = nq >= kQueryOrderMin;
   if (ordered) {
     const size_t nb = (size_t)d->nbins;
     if (ox.alloc(nq) != hipSuccess || oy.alloc(nq) != hipSuccess || oz.alloc(nq) != hipSuccess ||
         obins.alloc(nq) != hipSuccess || oorder.alloc(nq) != hipSuccess || ocnt.alloc(nb) != hipSuccess ||
-        odelim.alloc(nb + 1) != hipSuccess || ocursor.alloc(nb) != hipSuccess ||
+        odelim.alloc(nb + 1) != hipSuccess || orank.alloc(nq) != hipSuccess ||
         osums.alloc((nb + 1023) / 1024 + 1) != hipSuccess || omisc.alloc(4) != hipSuccess)
       return c->fail(TESS_E_NOMEM, "device allocation failed");
-    SortBufs b{obins.p, ocnt.p, odelim.p, ocursor.p, oorder.p, nullptr, osums.p, nullptr, omisc.p};
+    SortBufs b{obins.p, ocnt.p, odelim.p, oorder.p, orank.p, osums.p, nullptr, omisc.p};
     if ((st = c->hip(launch_soa(qd.p, (int)nq, ox.p, oy.p, oz.p, s), "query order")) != TESS_OK ||
         (st = c->hip(launch_grid_order(ox.p, oy.p, oz.p, (int)nq, d->grid.p, d->nbins, b, s), "query order")) !=
             TESS_OK)
@@ -141,7 +141,7 @@ tess_status query_impl(tess_diagram* d, int kind, const double* xyz, size_t nq, 
   a.sorted = d->sorted.p;
   a.delim = d->delim.p;
   a.pts = d->pts.p;
-  a.groups = target_group >= 0 ? d->groups.p : nullptr;
+  a.groups = target_group >= 0 ? d->sgroups.p : nullptr;
   a.target_group = target_group;
   a.q = qd.p;
   a.radius = rd.p;

@@ -1,18 +1,25 @@
 // query.hip -- radius queries over a diagram's grid (celery.rs:700-855,
 // :1023-1075; interface.rs:348-365).
 //
-// One wavefront per query, two passes over the same walk: the first counts
-// each query's results, a u64 scan turns the counts into CSR offsets, the
-// second writes the ids in the reference's order.  Box queries walk the index
-// box of the query in (i, j, k) loop order, 64 grid cells per step; the
-// neighbour cloud walks the shell table in canonical order, 64 entries per
-// step, until the first key above the radius.  The points of a step's cells
-// are then walked one per lane, so loads and stores of neighbouring lanes
-// are neighbouring addresses and a dense cell does not hold up the wave.
-// Large query sets are taken in grid order of their positions, so the
-// wavefronts running together read the same grid cells.  The walk is bound
-// by the reads of delimiters, sorted indices and (for the real radius)
-// gathered coordinates: integer and byte work on HBM.
+// Two passes over the same walk: the first counts each query's results, a
+// u64 scan turns the counts into CSR offsets, the second writes the ids in
+// the reference's order.
+//
+// Box queries walk the index box of the query in (i, j, k) loop order.  The
+// cells of a row (i, j) that the radius reaches are one interval of k (the
+// gap distance only grows away from the query's cell), and consecutive cells
+// are consecutive in the grid order, so a row is one run of points (or cell
+// ids) found from two delimiters.  The count pass gives a query 16 lanes, a
+// row each; the fill pass one wavefront.  The neighbour cloud walks the shell
+// table in canonical order, 64 entries per step, until the first key above
+// the radius.
+//
+// The points of a step's runs are walked one per lane, so loads and stores of
+// neighbouring lanes are neighbouring addresses.  Large query sets are taken
+// in grid order of their positions, so the wavefronts running together read
+// the same grid cells.  The walk is bound by the instructions around each 64
+// points and by the reads of delimiters, sorted indices and point records:
+// integer and byte work.
 #include "launch.h"
 #include "tess_internal.h"
 
@@ -45,6 +52,16 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// Lane l's value as a scalar.
+__device__ __forceinline__ uint32_t lane_u(uint32_t v, int l) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, l);
+}
+__device__ __forceinline__ double lane_d(double v, int l) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+  return __longlong_as_double(
+      (long long)(((unsigned long long)lane_u((uint32_t)(u >> 32), l) << 32) | lane_u((uint32_t)u, l)));
+}
+
 // Running maximum over the lanes (inclusive), values >= -1: DPP row shifts
 // inside the rows of 16, then row broadcasts (lanes without a source: -1).
 __device__ __forceinline__ int wave_max_scan(int v) {
@@ -74,31 +91,82 @@ __device__ __forceinline__ uint32_t wave_excl(uint32_t v, int lane, uint32_t* to
   return (uint32_t)x - v;
 }
 
-// The points of the step's 64 grid cells, in cell order and, inside a cell,
-// in grid (sorted-index) order: lane l's cell holds len points from grid
-// position s0 on (len 0: no cell).  The concatenation is walked 64 points at
-// a time, one point per lane; a lane finds its cell by binary search over the
-// cells' exclusive starts, read from their lanes.  MODE 0 keeps every point
+// Runs of at least this many points (on average over a step's runs) are
+// walked one by one by the whole wavefront: no search for a position's run,
+// but the last 64 of every run are part empty.  At 1M clustered points (290 a
+// run) the fill pass of 1M real-radius queries took 1.92 ms so and 2.45 ms
+// with the runs' concatenation searched; between 15 and 35 points a run the
+// two forms are within 5 %.
+constexpr uint32_t kRunWalkMin = 48;
+
+// The points of the step's 64 runs, in lane order: lane l's run holds len
+// points from grid position s0 on (len 0: none).  MODE 0 keeps every point
 // (only the count is needed in the count pass), MODE 1 the points within the
 // radius (celery.rs:700-702, :843-851), MODE 2 the points of the target group
-// (interface.rs:358-361); kept points are written in walk order (ballot rank).
+// (interface.rs:358-361), MODE 3 lists the positions themselves (cell ids);
+// kept points are written in walk order (ballot rank).  Long runs are walked
+// one after another; short ones as their concatenation, 64 positions at a
+// time, a lane finding its run from heads marked in LDS.
+template <int MODE>
+__device__ __forceinline__ bool keep_point(const QueryArgs& a, uint32_t s, double qx, double qy, double qz, double r2,
+                                           uint32_t& id) {
+  if (MODE == 3) {
+    id = s;
+    return true;
+  }
+  if (MODE == 1) {
+    const PointRec pr = a.pts[s];
+    id = pr.id;
+    const double dx = qx - pr.x, dy = qy - pr.y, dz = qz - pr.z;
+    return (dx * dx + dy * dy) + dz * dz <= r2;
+  }
+  id = a.sorted[s];
+  return MODE == 0 || a.groups[s] == a.target_group;
+}
+
 template <int MODE, bool FILL>
 __device__ __forceinline__ void emit_points(const QueryArgs& a, uint32_t s0, uint32_t len, int lane, double qx,
                                             double qy, double qz, double r2, uint64_t& cursor, uint64_t end,
                                             uint8_t* head) {
+  constexpr bool ALL = MODE == 0 || MODE == 3;
   uint32_t total;
   const uint32_t start = wave_excl(len, lane, &total);
-  if (MODE == 0 && !FILL) {
+  if (ALL && !FILL) {
     cursor += total;
     return;
   }
   const uint64_t below = (1ull << lane) - 1ull;
-  int carry = 0;  // the cell holding the last position of the previous window
+  const uint64_t runs = __ballot(len > 0);
+  if (total >= kRunWalkMin * (uint32_t)__popcll(runs)) {
+    for (uint64_t m = runs; m;) {
+      const int l = __builtin_ctzll(m);
+      m &= m - 1ull;
+      const uint32_t b = (uint32_t)__builtin_amdgcn_readlane((int)s0, l);
+      const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)len, l);
+      for (uint32_t p = (uint32_t)lane; p < n + (uint32_t)lane; p += 64) {  // whole wavefronts
+        uint32_t id = 0;
+        const bool keep = p < n && keep_point<MODE>(a, b + p, qx, qy, qz, r2, id);
+        if (ALL) {
+          if (keep && cursor + p < end) a.ids[cursor + p] = id;
+        } else {
+          const uint64_t km = __ballot(keep);
+          if (FILL && keep) {
+            const uint64_t pos = cursor + (uint64_t)__popcll(km & below);
+            if (pos < end) a.ids[pos] = id;
+          }
+          cursor += (uint64_t)__popcll(km);
+        }
+      }
+      if (ALL) cursor += n;
+    }
+    return;
+  }
+  int carry = 0;  // the run holding the last position of the previous window
   for (uint32_t base = 0; base < total; base += 64) {
     const uint32_t p = base + (uint32_t)lane;
-    // the cell of position p: the last non-empty cell starting at or before
-    // p (each writes its lane at its start in this window, then a running
-    // maximum; before the window's first start, the carried cell)
+    // the run of position p: the last non-empty one starting at or before p
+    // (each writes its lane at its start in this window, then a running
+    // maximum; before the window's first start, the carried run)
     head[lane] = 0xff;
     wave_sync();
     if (len > 0 && start >= base && start - base < 64u) head[start - base] = (uint8_t)lane;
@@ -109,25 +177,10 @@ __device__ __forceinline__ void emit_points(const QueryArgs& a, uint32_t s0, uin
     carry = __builtin_amdgcn_readlane(c, 63);
     wave_sync();
     const uint32_t cs0 = __shfl(s0, c, 64), cstart = __shfl(start, c, 64);
-    const bool valid = p < total;
-    const uint32_t s = cs0 + (p - cstart);
     uint32_t id = 0;
-    bool keep = false;
-    if (valid) {
-      if (MODE != 1) id = a.sorted[s];
-      if (MODE == 0) {
-        keep = true;
-      } else if (MODE == 1) {
-        const PointRec pr = a.pts[s];
-        id = pr.id;
-        const double dx = qx - pr.x, dy = qy - pr.y, dz = qz - pr.z;
-        keep = (dx * dx + dy * dy) + dz * dz <= r2;
-      } else {
-        keep = a.groups[id] == a.target_group;
-      }
-    }
-    if (MODE == 0) {
-      if (valid && cursor + p < end) a.ids[cursor + p] = id;
+    const bool keep = p < total && keep_point<MODE>(a, cs0 + (p - cstart), qx, qy, qz, r2, id);
+    if (ALL) {
+      if (keep && cursor + p < end) a.ids[cursor + p] = id;
     } else {
       const uint64_t m = __ballot(keep);
       if (FILL && keep) {
@@ -137,70 +190,205 @@ __device__ __forceinline__ void emit_points(const QueryArgs& a, uint32_t s0, uin
       cursor += (uint64_t)__popcll(m);
     }
   }
-  if (MODE == 0) cursor += total;
+  if (ALL) cursor += total;
+}
+
+// The index box of a query and its rows.
+struct QueryBox {
+  int i0, j0, k0, k1, hx, hy, hz;
+  uint32_t nj, rows;  // rows 0: nothing in reach
+  double r2;
+};
+
+__device__ __forceinline__ QueryBox query_box(const GridDev& G, double qx, double qy, double qz, double r) {
+  QueryBox q;
+  const int cpd = G.cpd;
+  q.i0 = q_axis_index(max_float(qx - r, G.xmin), G.xmin, G.xmax, G.ix, cpd);
+  q.j0 = q_axis_index(max_float(qy - r, G.ymin), G.ymin, G.ymax, G.iy, cpd);
+  q.k0 = q_axis_index(max_float(qz - r, G.zmin), G.zmin, G.zmax, G.iz, cpd);
+  const int i1 = q_axis_index(min_float(qx + r, G.xmax), G.xmin, G.xmax, G.ix, cpd);
+  const int j1 = q_axis_index(min_float(qy + r, G.ymax), G.ymin, G.ymax, G.iy, cpd);
+  q.k1 = q_axis_index(min_float(qz + r, G.zmax), G.zmin, G.zmax, G.iz, cpd);
+  q.hx = q_axis_index(qx, G.xmin, G.xmax, G.ix, cpd);
+  q.hy = q_axis_index(qy, G.ymin, G.ymax, G.iy, cpd);
+  q.hz = q_axis_index(qz, G.zmin, G.zmax, G.iz, cpd);
+  q.r2 = r * r;
+  const int ni = i1 - q.i0 + 1, nj = j1 - q.j0 + 1;
+  q.nj = nj > 0 ? (uint32_t)nj : 0u;
+  // a NaN radius admits no cell (ds <= NaN is false): skip the walk
+  q.rows = ni > 0 && nj > 0 && q.k1 >= q.k0 && r == r ? (uint32_t)ni * (uint32_t)nj : 0u;
+  return q;
+}
+
+// Row t of the box: its cells in reach are first .. first + count - 1.
+// celery.rs:708-743: the gap distance of the query's cell to (i, j, k) is
+// compared with the radius; along k it falls to the query's cell and rises
+// after it, so the reached cells are an interval, whose ends a bisection of
+// k0 .. hz and of hz .. k1 finds (the query's own k is reached if any is).
+// With a negative radius hz may lie outside k0 .. k1: then the interval is
+// bounded on the other side by the box.
+__device__ __forceinline__ uint32_t query_row(const GridDev& G, const QueryBox& q, uint32_t t, uint32_t& first) {
+  const int cpd = G.cpd;
+  const int i = q.i0 + (int)(t / q.nj), j = q.j0 + (int)(t % q.nj);
+  const double gx = (double)cell_gap(q.hx, i) * G.sx, gy = (double)cell_gap(q.hy, j) * G.sy;
+  const double g2 = gx * gx + gy * gy;
+  auto in = [&](int k) {
+    const double gz = (double)cell_gap(q.hz, k) * G.sz;
+    return g2 + gz * gz <= q.r2;
+  };
+  first = ((uint32_t)i * (uint32_t)cpd + (uint32_t)j) * (uint32_t)cpd;  // celery.rs:317-325
+  // the box's k nearest the query's
+  const int near = q.hz < q.k0 ? q.k0 : (q.hz > q.k1 ? q.k1 : q.hz);
+  if (!in(near)) return 0;
+  int ka = q.k0, kb = q.k1;
+  for (int hi = near; ka < hi;) {  // the smallest k in reach is in ka .. hi
+    const int mid = (ka + hi) >> 1;
+    if (in(mid))
+      hi = mid;
+    else
+      ka = mid + 1;
+  }
+  for (int lo = near; lo < kb;) {  // the largest is in lo .. kb
+    const int mid = (lo + kb + 1) >> 1;
+    if (in(mid))
+      lo = mid;
+    else
+      kb = mid - 1;
+  }
+  first += (uint32_t)ka;
+  return (uint32_t)(kb - ka + 1);
 }
 
 // find_cells_in_radius (KIND 0) and the two neighbour searches built on it
 // (KIND 1 cell radius, KIND 2 real radius): celery.rs:753-855.
+
+// Cells or points of every query's rows (unfiltered: an upper bound for KIND
+// 2), 16 lanes (a DPP row) per query, a row of the box each.  1M queries of
+// 10 cells: 120 us (one wavefront per query, a lane per cell: 450 us).
+template <int KIND>
+__global__ __launch_bounds__(256) void k_query_box_count(QueryArgs a) {
+  const int sub = threadIdx.x & 15;
+  const uint32_t w = blockIdx.x * 16u + (threadIdx.x >> 4);
+  const bool live = w < (uint32_t)a.nq;
+  const uint32_t qi = live ? (a.order ? a.order[w] : w) : 0u;
+  const double* p = a.q + 3 * (size_t)qi;
+  QueryBox q = query_box(a.g, p[0], p[1], p[2], a.radius[(size_t)qi * a.rstride]);
+  uint32_t sum = 0;
+  if (live)
+    for (uint32_t t = (uint32_t)sub; t < q.rows; t += 16) {
+      uint32_t first;
+      const uint32_t n = query_row(a.g, q, t, first);
+      if (n) sum += KIND == 0 ? n : a.delim[first + n] - a.delim[first];
+    }
+  int v = (int)sum;
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
+  if (live && sub == 15) a.count[qi] = (uint32_t)v;
+}
+
+// The ids (without FILL their exact number): 16 lanes per query, 16 rows of
+// the box per step, so that four queries share the instructions of the walk's
+// set-up.  Short rows are walked by the query's 16 lanes; when the step's rows
+// hold kRunWalkMin points or more on average, the whole wavefront takes them,
+// one query after the other, and reads 64 neighbouring points at a time.
+// a.count (nullable): ids per query.  Fill pass of 1M queries, one wavefront
+// per query over 64 cells a step before: real radius at clustered points (124
+// ids) 2.89 -> 1.63 ms, at uniform points (5 ids) 0.65 -> 0.29 ms; cell radius
+// at clustered points (1,183 ids) 2.49 -> 1.96 ms.
 template <int KIND, bool FILL>
 __global__ __launch_bounds__(256) void k_query_box(QueryArgs a) {
-  __shared__ uint8_t heads[4][64];
-  uint8_t* head = heads[threadIdx.x >> 6];
-  const int lane = threadIdx.x & 63;
-  const int w = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (w >= a.nq) return;
-  const int qi = a.order ? (int)a.order[w] : w;
-  const GridDev& G = a.g;
-  const int cpd = G.cpd;
+  constexpr int MODE = KIND == 0 ? 3 : (KIND == 1 ? 0 : 1);
+  constexpr bool ALL = MODE != 1;
+  constexpr int kAhead = 2;  // points of every lane in flight
+  const int lane = threadIdx.x & 63, sub = lane & 15, group = lane & 48;
+  const uint32_t w = blockIdx.x * 16u + (threadIdx.x >> 4);
+  const bool live = w < (uint32_t)a.nq;
+  const uint32_t qi = live ? (a.order ? a.order[w] : w) : 0u;
   const double qx = a.q[3 * (size_t)qi], qy = a.q[3 * (size_t)qi + 1], qz = a.q[3 * (size_t)qi + 2];
-  const double r = a.radius[(size_t)qi * a.rstride];
-  const int i0 = q_axis_index(max_float(qx - r, G.xmin), G.xmin, G.xmax, G.ix, cpd);
-  const int j0 = q_axis_index(max_float(qy - r, G.ymin), G.ymin, G.ymax, G.iy, cpd);
-  const int k0 = q_axis_index(max_float(qz - r, G.zmin), G.zmin, G.zmax, G.iz, cpd);
-  const int i1 = q_axis_index(min_float(qx + r, G.xmax), G.xmin, G.xmax, G.ix, cpd);
-  const int j1 = q_axis_index(min_float(qy + r, G.ymax), G.ymin, G.ymax, G.iy, cpd);
-  const int k1 = q_axis_index(min_float(qz + r, G.zmax), G.zmin, G.zmax, G.iz, cpd);
-  const int hx = q_axis_index(qx, G.xmin, G.xmax, G.ix, cpd);
-  const int hy = q_axis_index(qy, G.ymin, G.ymax, G.iy, cpd);
-  const int hz = q_axis_index(qz, G.zmin, G.zmax, G.iz, cpd);
-  const double r2 = r * r;
-  const int ni = i1 - i0 + 1, nj = j1 - j0 + 1, nk = k1 - k0 + 1;
-  const uint64_t njk = (uint64_t)(nj > 0 ? nj : 0) * (uint64_t)(nk > 0 ? nk : 0);
-  // a NaN radius admits no cell (ds <= NaN is false): skip the walk
-  const uint64_t total = (ni > 0 && r == r) ? (uint64_t)ni * njk : 0;
-  uint64_t cursor = FILL ? a.offsets[qi] : 0;
-  const uint64_t end = FILL ? a.offsets[qi + 1] : 0;
-  const uint64_t below = (1ull << lane) - 1ull;
-  for (uint64_t base = 0; base < total; base += 64) {
-    const uint64_t idx = base + (uint64_t)lane;
-    bool in = false;
-    uint32_t b = 0;
-    if (idx < total) {
-      const uint64_t rem = idx % njk;
-      const int i = i0 + (int)(idx / njk), j = j0 + (int)(rem / (uint64_t)nk), k = k0 + (int)(rem % (uint64_t)nk);
-      // celery.rs:708-743: gap distance of the query's cell to (i, j, k)
-      const double gx = (double)cell_gap(hx, i) * G.sx, gy = (double)cell_gap(hy, j) * G.sy,
-                   gz = (double)cell_gap(hz, k) * G.sz;
-      in = (gx * gx + gy * gy) + gz * gz <= r2;
-      b = ((uint32_t)i * (uint32_t)cpd + (uint32_t)j) * (uint32_t)cpd + (uint32_t)k;  // celery.rs:317-325
+  QueryBox q = query_box(a.g, qx, qy, qz, a.radius[(size_t)qi * a.rstride]);
+  if (!live) q.rows = 0;
+  const uint64_t begin = FILL ? a.offsets[qi] : 0;
+  const uint32_t room = FILL ? (uint32_t)(a.offsets[qi + 1] - begin) : 0u;
+  uint32_t cursor = 0;  // ids listed so far
+  for (uint32_t base = 0; __ballot(base < q.rows); base += 16) {
+    uint32_t s0 = 0, len = 0;
+    if (base < q.rows && (uint32_t)sub < q.rows - base) {
+      uint32_t first;
+      const uint32_t n = query_row(a.g, q, base + (uint32_t)sub, first);
+      if (KIND == 0) {
+        s0 = first;
+        len = n;
+      } else if (n) {
+        s0 = a.delim[first];
+        len = a.delim[first + n] - s0;
+      }
     }
-    if (KIND == 0) {
-      const uint64_t m = __ballot(in);
-      if (FILL && in) {
-        const uint64_t pos = cursor + (uint64_t)__popcll(m & below);
-        if (pos < end) a.ids[pos] = b;
+    const uint64_t all = __ballot(len > 0);
+    uint32_t total;
+    (void)wave_excl(len, lane, &total);
+    if (total >= kRunWalkMin * (uint32_t)__popcll(all)) {
+      for (int g = 0; g < 64; g += 16) {
+        uint32_t runs = (uint32_t)(all >> g) & 0xffffu;
+        if (!runs) continue;
+        const double gx = lane_d(qx, g), gy = lane_d(qy, g), gz = lane_d(qz, g), g2 = lane_d(q.r2, g);
+        const uint64_t gbegin = ((uint64_t)lane_u((uint32_t)(begin >> 32), g) << 32) | lane_u((uint32_t)begin, g);
+        const uint32_t groom = lane_u(room, g);
+        uint32_t at = lane_u(cursor, g);
+        uint32_t* ids = a.ids + gbegin;
+        for (; runs; runs &= runs - 1u) {
+          const int l = g + __builtin_ctz(runs);
+          const uint32_t b = lane_u(s0, l), n = lane_u(len, l);
+          for (uint32_t p0 = 0; p0 < n; p0 += 64) {
+            const uint32_t p = p0 + (uint32_t)lane;
+            uint32_t id = 0;
+            const bool keep = p < n && keep_point<MODE>(a, b + p, gx, gy, gz, g2, id);
+            if (ALL) {
+              if (keep && at + p < groom) ids[at + p] = id;
+            } else {
+              const uint64_t m = __ballot(keep);
+              const uint32_t pos = at + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+              if (FILL && keep && pos < groom) ids[pos] = id;
+              at += (uint32_t)__popcll(m);
+            }
+          }
+          if (ALL) at += n;
+        }
+        if (group == g) cursor = at;
       }
-      cursor += (uint64_t)__popcll(m);
-    } else {
-      uint32_t s0 = 0, len = 0;
-      if (in) {
-        s0 = a.delim[b];
-        len = a.delim[b + 1] - s0;
+      continue;
+    }
+    uint32_t* ids = a.ids + begin;
+    for (uint32_t runs = (uint32_t)(all >> group) & 0xffffu; runs; runs &= runs - 1u) {
+      const int l = group + __builtin_ctz(runs);
+      const uint32_t b = (uint32_t)__shfl((int)s0, l, 64), n = (uint32_t)__shfl((int)len, l, 64);
+      for (uint32_t p0 = 0; p0 < n; p0 += 16 * kAhead) {
+        uint32_t id[kAhead];
+        bool keep[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+          const uint32_t p = p0 + 16u * u + (uint32_t)sub;
+          id[u] = 0;
+          keep[u] = p < n && keep_point<MODE>(a, b + p, qx, qy, qz, q.r2, id[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+          if (ALL) {
+            const uint32_t pos = cursor + p0 + 16u * u + (uint32_t)sub;
+            if (keep[u] && pos < room) ids[pos] = id[u];
+          } else {
+            const uint32_t m = (uint32_t)(__ballot(keep[u]) >> group) & 0xffffu;
+            const uint32_t pos = cursor + (uint32_t)__popc(m & ((1u << sub) - 1u));
+            if (FILL && keep[u] && pos < room) ids[pos] = id[u];
+            cursor += (uint32_t)__popc(m);
+          }
+        }
       }
-      emit_points<KIND == 1 ? 0 : 1, FILL>(a, s0, len, lane, qx, qy, qz, r2, cursor, end, head);
+      if (ALL) cursor += n;
     }
   }
-  if (lane == 0 && a.count) a.count[qi] = (uint32_t)(FILL ? cursor - a.offsets[qi] : cursor);
+  if (live && sub == 0 && a.count) a.count[qi] = cursor;
 }
 
 // Cell::compute_neighbor_cloud: expand_all_in_radius from the query's grid
@@ -252,15 +440,22 @@ __global__ __launch_bounds__(256) void k_query_cloud(QueryArgs a) {
 template <bool FILL>
 hipError_t launch_query_pass(const QueryArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)((a.nq + 3) / 4)), block(256);
+  const dim3 grid16((unsigned)((a.nq + 15) / 16));
   switch (a.kind) {
     case 0:
-      hipLaunchKernelGGL((k_query_box<0, FILL>), grid, block, 0, s, a);
+      if (FILL)
+        hipLaunchKernelGGL((k_query_box<0, true>), grid16, block, 0, s, a);
+      else
+        hipLaunchKernelGGL((k_query_box_count<0>), grid16, block, 0, s, a);
       break;
     case 1:
-      hipLaunchKernelGGL((k_query_box<1, FILL>), grid, block, 0, s, a);
+      if (FILL)
+        hipLaunchKernelGGL((k_query_box<1, true>), grid16, block, 0, s, a);
+      else
+        hipLaunchKernelGGL((k_query_box_count<1>), grid16, block, 0, s, a);
       break;
     case 2:
-      hipLaunchKernelGGL((k_query_box<2, FILL>), grid, block, 0, s, a);
+      hipLaunchKernelGGL((k_query_box<2, FILL>), grid16, block, 0, s, a);
       break;
     default:
       hipLaunchKernelGGL((k_query_cloud<FILL>), grid, block, 0, s, a);

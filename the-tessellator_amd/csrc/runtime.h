@@ -192,11 +192,11 @@ struct tess_diagram {
   bool have_groups = false;
   // inputs
   DevBuf<double> x, y, z, xyz_tmp;
-  DevBuf<int64_t> groups;
+  DevBuf<int64_t> groups, sgroups;  // by point, and in grid order (set by the binning)
   // grid
   DevBuf<GridDev> grid;
   DevBuf<double> part;
-  DevBuf<uint32_t> bins, cnt, delim, cursor, sorted, scratch, sums, big, misc, inv;
+  DevBuf<uint32_t> bins, cnt, delim, sorted, scratch, sums, big, misc, inv;
   DevBuf<PointRec> pts;    // points in grid order
   DevBuf<uint32_t> codes;  // Morton codes (TESS_ORDER_MORTON)
   GridDev hgrid;
@@ -235,7 +235,7 @@ struct tess_diagram {
   // freed with the diagram): the per-query counts and their scans, the
   // grid order of large query sets, the kept ids' upper-bound slots
   struct {
-    DevBuf<uint32_t> cnt, obins, ocnt, odelim, ocursor, oorder, osums, omisc, slots;
+    DevBuf<uint32_t> cnt, obins, ocnt, odelim, orank, oorder, osums, omisc, slots;
     DevBuf<uint64_t> sums, boff;
     DevBuf<double> ox, oy, oz;
   } qtmp;

@@ -114,7 +114,7 @@ struct CellArgs {
                            // then index these sites and the outputs
                            // (Diagram::get_cell_at_particle, no self)
   int xcd_chunk;           // > 0: XCDs take runs of this many consecutive cells
-  const int64_t* groups;   // nullable
+  const int64_t* groups;   // in grid order; nullable
   int64_t target_group;    // < 0: none
   double radius_limit;     // NaN: none (expand_all_in_radius cut-off otherwise)
   // outputs, indexed by original point index
@@ -197,7 +197,7 @@ struct QueryArgs {
   const uint32_t* sorted;  // grid-ordered point ids [n]
   const uint32_t* delim;   // [cpd^3 + 1]
   const PointRec* pts;     // points in grid order
-  const int64_t* groups;   // by point id; null: no group filter
+  const int64_t* groups;   // in grid order; null: no group filter
   int64_t target_group;
   const double* q;         // query positions, AoS [3 nq]
   const uint32_t* order;   // nullable: wavefront w takes query order[w]
