@@ -466,17 +466,29 @@ hipError_t launch_query_pass(const QueryArgs& a, hipStream_t s) {
 
 }  // namespace
 
-// Ids of query q from src[from[q] ..] to dst[to[q] .. to[q + 1]), one
-// wavefront per query.
+// Ids of query q from src[from[q] ..] to dst[to[q] .. to[q + 1]): 16 lanes per
+// query, eight ids of every lane in flight.  124 ids for each of 1M queries:
+// 500 -> 259 us (one wavefront per query, one id of a lane at a time).
 __global__ __launch_bounds__(256) void k_query_compact(int nq, const uint64_t* __restrict__ from,
                                                        const uint64_t* __restrict__ to,
                                                        const uint32_t* __restrict__ src,
                                                        uint32_t* __restrict__ dst) {
-  const int lane = threadIdx.x & 63;
-  const int q = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (q >= nq) return;
-  const uint64_t f = from[q], t = to[q], m = to[q + 1] - t;
-  for (uint64_t k = lane; k < m; k += 64) dst[t + k] = src[f + k];
+  constexpr int kAhead = 8;
+  const int sub = threadIdx.x & 15;
+  const uint32_t q = blockIdx.x * 16u + (threadIdx.x >> 4);
+  if (q >= (uint32_t)nq) return;
+  const uint64_t t = to[q], m = to[q + 1] - t;
+  src += from[q];
+  dst += t;
+  for (uint64_t k0 = (uint64_t)sub; k0 < m; k0 += 16 * kAhead) {
+    uint32_t v[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u)
+      if (k0 + 16 * u < m) v[u] = src[k0 + 16 * u];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u)
+      if (k0 + 16 * u < m) dst[k0 + 16 * u] = v[u];
+  }
 }
 
 hipError_t launch_query_count(const QueryArgs& a, hipStream_t s) { return launch_query_pass<false>(a, s); }
@@ -484,7 +496,7 @@ hipError_t launch_query_fill(const QueryArgs& a, hipStream_t s) { return launch_
 hipError_t launch_query_compact(int nq, const uint64_t* from, const uint64_t* to, const uint32_t* src, uint32_t* dst,
                                 hipStream_t s) {
   if (nq <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_query_compact, dim3((unsigned)((nq + 3) / 4)), dim3(256), 0, s, nq, from, to, src, dst);
+  hipLaunchKernelGGL(k_query_compact, dim3((unsigned)((nq + 15) / 16)), dim3(256), 0, s, nq, from, to, src, dst);
   return hipGetLastError();
 }
 
