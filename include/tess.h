@@ -146,6 +146,9 @@ typedef struct {
 void tess_opts_default(tess_opts* opts);
 
 /* ---- context ---------------------------------------------------------- */
+/* Large device blocks (2 MiB and more) of destroyed objects are kept for the
+ * next ones, at most 1/64 of the device's memory; destroying the last context
+ * on the device gives them all back. */
 tess_status tess_ctx_create(int hip_device, tess_ctx** out);
 void tess_ctx_destroy(tess_ctx* ctx);
 const char* tess_last_error(const tess_ctx* ctx);

@@ -569,6 +569,7 @@ tess_status tess_ctx_create(int dev, tess_ctx** out) {
     delete c;
     return TESS_E_DEVICE;
   }
+  pool_context_add(dev);
   *out = c;
   return TESS_OK;
 }
@@ -580,7 +581,9 @@ void tess_ctx_destroy(tess_ctx* c) {
   c->tables.clear();
   c->diag.reset();
   (void)hipStreamDestroy(c->stream);
+  const int device = c->device;
   delete c;
+  pool_context_remove(device);
 }
 
 const char* tess_last_error(const tess_ctx* c) { return c ? c->err.c_str() : "null context"; }

@@ -46,6 +46,7 @@ hipError_t grow(DevBuf<T>& b, size_t need, size_t keep, hipStream_t s) {
   }
   std::swap(b.p, nb.p);
   std::swap(b.n, nb.n);
+  std::swap(b.block, nb.block);
   return hipSuccess;
 }
 

@@ -18,6 +18,21 @@
 
 namespace tess {
 
+// Large device blocks, kept between objects (pool.cpp).  pool_alloc allocates
+// on the current device; pool_free waits for the device's work, like hipFree.
+struct PoolBlock {
+  void* p = nullptr;
+  void* token = nullptr;
+  size_t bytes = 0;
+  int device = -1;
+};
+constexpr size_t kPoolMin = size_t(2) << 20;  // smaller ones the runtime suballocates
+hipError_t pool_alloc(size_t bytes, PoolBlock* out);
+void pool_free(const PoolBlock& b);
+// contexts on a device: with the last one its kept blocks go
+void pool_context_add(int device);
+void pool_context_remove(int device);
+
 template <class T>
 struct DevBuf {
   T* p = nullptr;
@@ -26,9 +41,15 @@ struct DevBuf {
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
   bool own = true;  // false: a view into memory owned elsewhere
+  PoolBlock block;  // from kPoolMin bytes on
   ~DevBuf() { reset(); }
   void reset() {
-    if (p && own) (void)hipFree(p);
+    if (block.p) {
+      pool_free(block);
+      block = PoolBlock{};
+    } else if (p && own) {
+      (void)hipFree(p);
+    }
     p = nullptr;
     n = 0;
     own = true;
@@ -43,7 +64,13 @@ struct DevBuf {
     if (count <= n && p) return hipSuccess;
     reset();
     if (count == 0) count = 1;
-    hipError_t e = hipMalloc((void**)&p, sizeof(T) * count);
+    hipError_t e;
+    if (sizeof(T) * count >= kPoolMin) {
+      e = pool_alloc(sizeof(T) * count, &block);
+      p = static_cast<T*>(block.p);
+    } else {
+      e = hipMalloc((void**)&p, sizeof(T) * count);
+    }
     if (e == hipSuccess) n = count;
     return e;
   }
