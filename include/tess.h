@@ -180,10 +180,10 @@ tess_status tess_diagram_compute(tess_diagram* d);
 tess_status tess_diagram_total_faces(const tess_diagram* d, uint64_t* out);
 /* Copy results to host arrays: volume[n], face_count[n], face_offset[n+1],
  * neighbor[total_faces], face_area[total_faces]; any pointer may be NULL.
- * Arrays of 16 MiB or more (here and in every other *_copy* call) come down
- * through two 64 MiB pinned host buffers the context allocates on first use
- * and keeps until tess_ctx_destroy, copied out by up to eight host threads;
- * calls on one context take the buffers in turn. */
+ * The arrays of a call (here and in the other *_copy* calls) come down
+ * together through two pinned host buffers of 1 to 64 MiB that the context
+ * allocates when they are needed and keeps until tess_ctx_destroy, copied out
+ * by up to eight host threads; calls on one context take the buffers in turn. */
 tess_status tess_diagram_copy_cells(const tess_diagram* d, double* volume, uint32_t* face_count,
                                     uint64_t* face_offset, int32_t* neighbor, double* face_area);
 tess_status tess_diagram_device_cells(const tess_diagram* d, tess_cells_device* out);

@@ -141,38 +141,84 @@ void host_copy(char* dst, const char* src, size_t len) {
   for (auto& x : th) x.join();
 }
 
-hipError_t download(tess_ctx* c, void* dst, const void* src, size_t bytes) {
-  constexpr size_t kMin = size_t(16) << 20;
-  if (bytes < kMin) return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
-  // at least four chunks (so that transfers and host copies overlap), of
-  // 8 MiB to one staging buffer each
-  const size_t kChunk = std::min(Staging::kBytes, std::max(size_t(8) << 20, (bytes / 4 + 4095) & ~size_t(4095)));
+namespace {
+
+// Without pinned memory: plain copies.
+hipError_t download_plain(const Piece* pieces, int count) {
+  for (int k = 0; k < count; ++k) {
+    const Piece& p = pieces[k];
+    if (!p.dst || !p.bytes) continue;
+    hipError_t e = hipMemcpy(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost);
+    uint64_t m = 0;
+    if (e == hipSuccess && p.sub) e = hipMemcpy(&m, p.sub, 8, hipMemcpyDeviceToHost);
+    if (e != hipSuccess) return e;
+    if (p.sub)
+      for (size_t i = 0; i < p.bytes / 8; ++i) static_cast<uint64_t*>(p.dst)[i] -= m;
+  }
+  return hipSuccess;
+}
+
+}  // namespace
+
+hipError_t download(tess_ctx* c, const Piece* pieces, int count) {
+  CopyOut a;
+  std::memset(&a, 0, sizeof(a));
+  char* out[kCopyOutPieces];
+  uint64_t total = 0;
+  for (int k = 0; k < count; ++k) {
+    if (!pieces[k].dst || !pieces[k].bytes) continue;
+    if (a.npieces == kCopyOutPieces) return hipErrorInvalidValue;
+    out[a.npieces] = static_cast<char*>(pieces[k].dst);
+    a.piece[a.npieces++] = {pieces[k].src, pieces[k].sub, total, pieces[k].bytes};
+    total += (pieces[k].bytes + 15) & ~size_t(15);
+  }
+  if (!total) return hipSuccess;
+  // one chunk up to 1 MiB, else four and more of 1 to 64 MiB: transfers and
+  // host copies overlap
+  constexpr size_t kOne = size_t(1) << 20;
+  const size_t chunk =
+      total <= kOne ? total : std::min(Staging::kBytes, std::max(kOne, (total / 4 + 4095) & ~size_t(4095)));
   Staging& S = c->stage;
   std::lock_guard<std::mutex> g(S.mu);
-  for (int k = 0; k < 2; ++k) {
-    if (!S.buf[k] && hipHostMalloc(&S.buf[k], Staging::kBytes, hipHostMallocDefault) != hipSuccess) {
-      S.buf[k] = nullptr;
-      return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);  // no pinned memory: the plain copy
+  for (int k = 0; k < (total > chunk ? 2 : 1); ++k) {
+    if (S.cap[k] < chunk) {
+      if (S.buf[k]) (void)hipHostFree(S.buf[k]);
+      size_t cap = kOne;
+      while (cap < chunk) cap *= 2;
+      S.cap[k] = 0;
+      if (hipHostMalloc(&S.buf[k], cap, hipHostMallocCoherent) != hipSuccess) {
+        S.buf[k] = nullptr;
+        return download_plain(pieces, count);
+      }
+      S.cap[k] = cap;
     }
-    if (!S.ev[k] && hipEventCreateWithFlags(&S.ev[k], hipEventDisableTiming) != hipSuccess) {
-      S.ev[k] = nullptr;
-      return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
+    if (!S.ev[k]) {
+      if (hipEventCreateWithFlags(&S.ev[k], hipEventDisableTiming) != hipSuccess) {
+        S.ev[k] = nullptr;
+        return download_plain(pieces, count);
+      }
     }
   }
-  const size_t nch = (bytes + kChunk - 1) / kChunk;
-  auto len_of = [&](size_t i) { return std::min(kChunk, bytes - i * kChunk); };
+  const size_t nch = (total + chunk - 1) / chunk;
   // chunk i goes to buffer i & 1; chunk i + 1 is issued before chunk i is
   // copied out, into the buffer chunk i - 1 left (copied out already)
   auto issue = [&](size_t i) {
-    hipError_t e = hipMemcpyAsync(S.buf[i & 1], static_cast<const char*>(src) + i * kChunk, len_of(i),
-                                  hipMemcpyDeviceToHost, c->stream);
+    a.base = i * chunk;
+    a.len = std::min<uint64_t>(chunk, total - a.base);
+    a.dst = S.buf[i & 1];
+    const hipError_t e = launch_copy_out(a, c->stream);
     return e == hipSuccess ? hipEventRecord(S.ev[i & 1], c->stream) : e;
   };
   hipError_t e = issue(0);
   for (size_t i = 0; i < nch && e == hipSuccess; ++i) {
     if (i + 1 < nch && (e = issue(i + 1)) != hipSuccess) break;
     if ((e = hipEventSynchronize(S.ev[i & 1])) != hipSuccess) break;
-    host_copy(static_cast<char*>(dst) + i * kChunk, static_cast<const char*>(S.buf[i & 1]), len_of(i));
+    const uint64_t lo = i * chunk, hi = std::min<uint64_t>(lo + chunk, total);
+    for (int k = 0; k < a.npieces; ++k) {
+      const CopyOutPiece& p = a.piece[k];
+      const uint64_t f = std::max(lo, p.start), t = std::min(hi, p.start + p.bytes);
+      if (f < t) host_copy(out[k] + (f - p.start), static_cast<const char*>(S.buf[i & 1]) + (f - lo), t - f);
+    }
   }
   if (e != hipSuccess) (void)hipStreamSynchronize(c->stream);  // nothing left in flight into the staging
   return e;
@@ -195,7 +241,7 @@ tess_status alloc_all(tess_diagram* d) {
             d->fcount.alloc(n) == hipSuccess && d->status.alloc(n) == hipSuccess &&
             d->redo.alloc(n + 1) == hipSuccess && d->snbr.alloc(arena_capacity(n)) == hipSuccess &&
             d->sarea.alloc(arena_capacity(n)) == hipSuccess && d->foff.alloc(n + 1) == hipSuccess &&
-            d->fsums.alloc((n + 1023) / 1024 + 1) == hipSuccess && d->work1.alloc(1) == hipSuccess &&
+            d->fsums.alloc((n + 1023) / 1024 + 1) == hipSuccess &&
             d->summary.alloc(kSummarySlots) == hipSuccess && d->tredo.alloc(n + 1) == hipSuccess &&
             d->spill.alloc(n + 1) == hipSuccess && d->fpos.alloc(n) == hipSuccess &&
             d->arena_ctr.alloc(kArenaWords) == hipSuccess;
@@ -684,13 +730,12 @@ tess_status tess_diagram_copy_cells(const tess_diagram* d, double* volume, uint3
   tess_ctx* c = d->ctx;
   (void)hipSetDevice(c->device);
   const size_t n = d->n;
-  hipError_t e = hipSuccess;
-  if (volume && e == hipSuccess) e = download(c, volume, d->volume.p, 8 * n);
-  if (fc && e == hipSuccess) e = download(c, fc, d->fcount.p, 4 * n);
-  if (fo && e == hipSuccess) e = download(c, fo, d->foff.p, 8 * (n + 1));
-  if (nbr && e == hipSuccess && d->total_faces) e = download(c, nbr, d->nbr.p, 4 * d->total_faces);
-  if (area && e == hipSuccess && d->total_faces) e = download(c, area, d->area.p, 8 * d->total_faces);
-  return c->hip(e, "download");
+  const Piece p[5] = {{volume, d->volume.p, 8 * n},
+                      {fc, d->fcount.p, 4 * n},
+                      {fo, d->foff.p, 8 * (n + 1)},
+                      {nbr, d->nbr.p, 4 * d->total_faces},
+                      {area, d->area.p, 8 * d->total_faces}};
+  return c->hip(download(c, p, 5), "download");
 }
 
 tess_status tess_diagram_device_cells(const tess_diagram* d, tess_cells_device* out) {
@@ -795,7 +840,7 @@ namespace {
 
 // One cell with its geometry through the single-cell export of the cell
 // kernel: the point `index` of the diagram, or the outside site `site`
-// (host, 3 doubles; index ignored).  Capacity 128 first, then 256.
+// (host, 3 doubles; index ignored).  Capacity 64 first, then 128 and 256.
 tess_status single_cell(tess_diagram* d, size_t index, const double* site, double search_radius,
                         int64_t target_group, tess_cell** out) {
   if (!d || !out) return TESS_E_INVALID;
@@ -846,9 +891,13 @@ tess_status single_cell(tess_diagram* d, size_t index, const double* site, doubl
   std::unique_ptr<tess_cell> cell(new (std::nothrow) tess_cell);
   if (!cell) return c->fail(TESS_E_NOMEM, "host allocation failed");
   uint32_t status = 0;
-  // capacity 128, then 256; a security ball past the shell table takes a
-  // table twice as long, up to the full order
-  int L = kTableL, vpl = 2;
+  // capacity 64, then 128 and 256; a security ball past the shell table takes
+  // a table twice as long, up to the full order.  A cell of a 100k set: 75 us
+  // at capacity 128, 50 at 64, so the larger ones are only reruns.
+  int L = kTableL, vpl = 1;
+  uint32_t fcst[2] = {0, 0};  // face count, status
+  std::vector<int32_t> nb(kFaceStage), ring(kFaceStage * 64), meta(2 + 256);
+  std::vector<double> ar(kFaceStage), vv(3 * 256);
   for (;;) {
     Table* t = c->table(d->cpd, G.sx, G.sy, G.sz, L, &st);
     if (!t) return st;
@@ -856,7 +905,7 @@ tess_status single_cell(tess_diagram* d, size_t index, const double* site, doubl
     a.fpos = nullptr;
     a.arena_next = nullptr;
     a.summary = nullptr;
-    a.work = site ? nullptr : d->work1.p;
+    a.work = site ? nullptr : d->inv.p + oi;
     a.ext = site ? d->one_site.p : nullptr;
     a.nwork = 1;
     a.xcd_chunk = 0;
@@ -873,14 +922,20 @@ tess_status single_cell(tess_diagram* d, size_t index, const double* site, doubl
     a.exp_meta = d->exp_meta.p;
     a.redo = nullptr;
     a.nredo = nullptr;
-    if ((!site && (st = c->hip(hipMemcpyAsync(d->work1.p, d->inv.p + oi, 4, hipMemcpyDeviceToDevice, s), "copy")) !=
-                      TESS_OK) ||
-        (st = c->hip(launch_cells(vpl, a, s), "cell kernel")) != TESS_OK ||
-        (st = c->hip(hipMemcpyAsync(&status, d->one_u32.p + 1, 4, hipMemcpyDeviceToHost, s), "copy")) != TESS_OK ||
-        (st = c->hip(hipStreamSynchronize(s), "cell kernel")) != TESS_OK)
+    // the status and everything read from a finished cell in one download
+    const Piece p[7] = {{fcst, d->one_u32.p, 8},
+                        {&cell->volume, d->one_vol.p, 8},
+                        {nb.data(), d->one_nbr.p, 4 * nb.size()},
+                        {ar.data(), d->one_area.p, 8 * ar.size()},
+                        {meta.data(), d->exp_meta.p, 4 * (size_t)(2 + 64 * vpl)},
+                        {vv.data(), d->exp_v.p, 24 * (size_t)(64 * vpl)},
+                        {ring.data(), d->exp_ring.p, 4 * ring.size()}};
+    if ((st = c->hip(launch_cells(vpl, a, s), "cell kernel")) != TESS_OK ||
+        (st = c->hip(download(c, p, 7), "cell kernel")) != TESS_OK)
       return st;
+    status = fcst[1];
     if ((status & TESS_CELL_CAPACITY) && vpl < 4)
-      vpl = 4;
+      vpl *= 2;
     else if ((status & TESS_CELL_TABLE) && L < d->cpd - 1)
       L = (int)std::min<int64_t>(2 * (int64_t)L, d->cpd - 1);
     else
@@ -890,17 +945,7 @@ tess_status single_cell(tess_diagram* d, size_t index, const double* site, doubl
     return c->fail(status & TESS_CELL_DEGENERATE ? TESS_E_DEGENERATE : TESS_E_CAPACITY,
                    (site ? std::string("the site's cell") : "cell " + std::to_string(index)) + " failed (status " +
                        std::to_string(status) + ")");
-  uint32_t fc = 0;
-  std::vector<int32_t> nb(kFaceStage), ring(kFaceStage * 64), meta(2 + 256);
-  std::vector<double> ar(kFaceStage), vv(3 * 256);
-  hipError_t e = hipMemcpy(&cell->volume, d->one_vol.p, 8, hipMemcpyDeviceToHost);
-  if (e == hipSuccess) e = hipMemcpy(&fc, d->one_u32.p, 4, hipMemcpyDeviceToHost);
-  if (e == hipSuccess) e = hipMemcpy(nb.data(), d->one_nbr.p, 4 * kFaceStage, hipMemcpyDeviceToHost);
-  if (e == hipSuccess) e = hipMemcpy(ar.data(), d->one_area.p, 8 * kFaceStage, hipMemcpyDeviceToHost);
-  if (e == hipSuccess) e = hipMemcpy(ring.data(), d->exp_ring.p, 4 * ring.size(), hipMemcpyDeviceToHost);
-  if (e == hipSuccess) e = hipMemcpy(meta.data(), d->exp_meta.p, 4 * meta.size(), hipMemcpyDeviceToHost);
-  if (e == hipSuccess) e = hipMemcpy(vv.data(), d->exp_v.p, 8 * vv.size(), hipMemcpyDeviceToHost);
-  if (e != hipSuccess) return c->hip(e, "download");
+  const uint32_t fc = fcst[0];
   cell->original = site ? -1 : (int64_t)index;  // Cell::original_index: None for a site
   const int vc = meta[0];
   for (uint32_t f = 0; f < fc; ++f) {

@@ -81,10 +81,13 @@ struct tess_batch {
   DevBuf<unsigned long long> arena;
   Mail* mail = nullptr;       // pinned
   GridDev* hgrid_pin = nullptr;  // pinned, nsets
+  DevBuf<uint64_t> fbase_dev;      // first face of each set, nsets + 1
+  uint64_t* fbase_pin = nullptr;   // the same, pinned
   uint64_t table_reruns = 0, spill_cells = 0;
   ~tess_batch() {
     if (mail) (void)hipHostFree(mail);
     if (hgrid_pin) (void)hipHostFree(hgrid_pin);
+    if (fbase_pin) (void)hipHostFree(fbase_pin);
   }
   DevBuf<tess_cell_stats> stats;
   DevBuf<SummarySlot> summary;  // kSummarySlots, shared by the sets
@@ -518,7 +521,11 @@ tess_status batch_compute(tess_batch* b, const tess_model* m) {
       TESS_OK)
     return st;
   (void)hipEventRecord(ev[3], s);
-  if ((st = c->hip(hipMemcpyAsync(&mail->total, b->foff.p + b->N, 8, hipMemcpyDeviceToHost, s), "total")) !=
+  if ((st = c->hip(launch_pick_u64(b->foff.p, b->base_dev.p, (int)b->nsets + 1, b->fbase_dev.p, s), "pick")) !=
+          TESS_OK ||
+      (st = c->hip(hipMemcpyAsync(b->fbase_pin, b->fbase_dev.p, 8 * (b->nsets + 1), hipMemcpyDeviceToHost, s),
+                   "set faces")) != TESS_OK ||
+      (st = c->hip(hipMemcpyAsync(&mail->total, b->foff.p + b->N, 8, hipMemcpyDeviceToHost, s), "total")) !=
           TESS_OK ||
       (st = c->hip(hipMemcpyAsync(&mail->arena, b->arena.p + (size_t)kArenaStride * (kArenaParts + 1), 8, hipMemcpyDeviceToHost, s),
                    "arena")) != TESS_OK ||
@@ -647,7 +654,9 @@ tess_status tess_batch_create(tess_ctx* ctx, size_t nsets, const double* const* 
             b->ctrl.alloc(kCtrlWords) == hipSuccess && b->fpos.alloc(N) == hipSuccess &&
             b->tredo.alloc(N) == hipSuccess && b->spill.alloc(N) == hipSuccess && b->arena.alloc(kArenaWords) == hipSuccess &&
             hipHostMalloc((void**)&b->mail, sizeof(Mail), hipHostMallocDefault) == hipSuccess &&
-            hipHostMalloc((void**)&b->hgrid_pin, sizeof(GridDev) * nsets, hipHostMallocDefault) == hipSuccess;
+            hipHostMalloc((void**)&b->hgrid_pin, sizeof(GridDev) * nsets, hipHostMallocDefault) == hipSuccess &&
+            hipHostMalloc((void**)&b->fbase_pin, 8 * (nsets + 1), hipHostMallocDefault) == hipSuccess &&
+            b->fbase_dev.alloc(nsets + 1) == hipSuccess;
   if (ok && b->opts.collect_stats) ok = b->stats.alloc(N) == hipSuccess;
   if (!ok) return ctx->fail(TESS_E_NOMEM, "device allocation failed");
   // points: one AoS upload, one SoA pass
@@ -799,13 +808,8 @@ tess_status tess_batch_total_faces(const tess_batch* b, size_t set, uint64_t* ou
   if (!b || !out) return TESS_E_INVALID;
   if (set >= b->nsets) return b->ctx->fail(TESS_E_INVALID, "set index out of range");
   if (!b->computed) return b->ctx->fail(TESS_E_STATE, "results read before compute");
-  uint64_t f[2];
-  (void)hipSetDevice(b->ctx->device);
-  tess_status st = b->ctx->hip(hipMemcpy(&f[0], b->foff.p + b->pbase[set], 8, hipMemcpyDeviceToHost), "download");
-  if (st == TESS_OK)
-    st = b->ctx->hip(hipMemcpy(&f[1], b->foff.p + b->pbase[set] + b->n[set], 8, hipMemcpyDeviceToHost), "download");
-  if (st == TESS_OK) *out = f[1] - f[0];
-  return st;
+  *out = b->fbase_pin[set + 1] - b->fbase_pin[set];
+  return TESS_OK;
 }
 
 tess_status tess_batch_copy_cells(const tess_batch* b, size_t set, double* volume, uint32_t* fc, uint64_t* fo,
@@ -816,16 +820,13 @@ tess_status tess_batch_copy_cells(const tess_batch* b, size_t set, double* volum
   if (!b->computed) return c->fail(TESS_E_STATE, "results read before compute");
   (void)hipSetDevice(c->device);
   const size_t p = b->pbase[set], n = b->n[set];
-  std::vector<uint64_t> off(n + 1);
-  hipError_t e = hipMemcpy(off.data(), b->foff.p + p, 8 * (n + 1), hipMemcpyDeviceToHost);
-  const uint64_t f0 = off[0], nf = off[n] - off[0];
-  if (e == hipSuccess && volume) e = download(c, volume, b->volume.p + p, 8 * n);
-  if (e == hipSuccess && fc) e = download(c, fc, b->fcount.p + p, 4 * n);
-  if (e == hipSuccess && fo)
-    for (size_t i = 0; i <= n; ++i) fo[i] = off[i] - f0;
-  if (e == hipSuccess && nbr && nf) e = download(c, nbr, b->nbr.p + f0, 4 * nf);
-  if (e == hipSuccess && area && nf) e = download(c, area, b->area.p + f0, 8 * nf);
-  return c->hip(e, "download");
+  const uint64_t f0 = b->fbase_pin[set], nf = b->fbase_pin[set + 1] - f0;
+  const Piece a[5] = {{volume, b->volume.p + p, 8 * n},
+                      {fc, b->fcount.p + p, 4 * n},
+                      {fo, b->foff.p + p, 8 * (n + 1), b->foff.p + p},  // from the set's first face
+                      {nbr, b->nbr.p + f0, 4 * nf},
+                      {area, b->area.p + f0, 8 * nf}};
+  return c->hip(download(c, a, 5), "download");
 }
 
 tess_status tess_batch_timings(const tess_batch* b, tess_timings* out) {

@@ -72,6 +72,26 @@ hipError_t launch_compact(const uint32_t* fcount, const uint64_t* foff, int n, c
                           const uint64_t* fpos = nullptr);
 hipError_t launch_invert(const uint32_t* sorted, int n, uint32_t* inv, hipStream_t s);
 
+// copyout.hip: bytes [base, base + len) of the pieces laid end to end, each
+// from a multiple of 16 (start), into dst (pinned host memory, 16-byte
+// aligned; len bytes rounded up to 16 are written).  sub: every uint64 of the
+// piece minus *sub.
+struct CopyOutPiece {
+  const void* src;
+  const uint64_t* sub;
+  uint64_t start, bytes;
+};
+constexpr int kCopyOutPieces = 8;
+struct CopyOut {
+  CopyOutPiece piece[kCopyOutPieces];
+  int npieces;
+  uint64_t base, len;
+  void* dst;
+};
+hipError_t launch_copy_out(const CopyOut& a, hipStream_t s);
+// out[k] = src[at[k]], k < n
+hipError_t launch_pick_u64(const uint64_t* src, const uint64_t* at, int n, uint64_t* out, hipStream_t s);
+
 // cell.hip: vpl = vertex slots per lane (1, 2 or 4)
 hipError_t launch_cells(int vpl, const CellArgs& a, hipStream_t s);
 // the same cells staging their geometry (CellArgs::geo_*), with the cell

@@ -209,14 +209,13 @@ tess_status tess_site_cells_copy(const tess_site_cells* p, double* volume, uint3
                                  uint64_t* face_offset, int32_t* neighbor, double* face_area) {
   if (!p) return TESS_E_INVALID;
   (void)hipSetDevice(p->ctx->device);
-  hipError_t e = hipSuccess;
   tess_ctx* c = p->ctx;
-  if (volume) e = download(c, volume, p->volume.p, 8 * p->m);
-  if (face_count && e == hipSuccess) e = download(c, face_count, p->fcount.p, 4 * p->m);
-  if (face_offset && e == hipSuccess) e = download(c, face_offset, p->foff.p, 8 * (p->m + 1));
-  if (neighbor && p->total && e == hipSuccess) e = download(c, neighbor, p->nbr.p, 4 * p->total);
-  if (face_area && p->total && e == hipSuccess) e = download(c, face_area, p->area.p, 8 * p->total);
-  return p->ctx->hip(e, "download");
+  const Piece a[5] = {{volume, p->volume.p, 8 * p->m},
+                      {face_count, p->fcount.p, 4 * p->m},
+                      {face_offset, p->foff.p, 8 * (p->m + 1)},
+                      {neighbor, p->nbr.p, 4 * p->total},
+                      {face_area, p->area.p, 8 * p->total}};
+  return c->hip(download(c, a, 5), "download");
 }
 
 tess_status tess_site_cells_copy_stats(const tess_site_cells* p, tess_cell_stats* stats) {

@@ -253,10 +253,8 @@ tess_status tess_query_timings(const tess_query* q, double ms[3]) {
 tess_status tess_query_copy(const tess_query* q, uint64_t* offsets, uint32_t* ids) {
   if (!q) return TESS_E_INVALID;
   (void)hipSetDevice(q->ctx->device);
-  hipError_t e = hipSuccess;
-  if (offsets) e = download(q->ctx, offsets, q->offsets.p, 8 * (q->nq + 1));
-  if (ids && q->total && e == hipSuccess) e = download(q->ctx, ids, q->ids.p, 4 * q->total);
-  return q->ctx->hip(e, "download");
+  const Piece p[2] = {{offsets, q->offsets.p, 8 * (q->nq + 1)}, {ids, q->ids.p, 4 * q->total}};
+  return q->ctx->hip(download(q->ctx, p, 2), "download");
 }
 
 tess_status tess_query_device(const tess_query* q, const uint64_t** offsets, const uint32_t** ids) {

@@ -96,12 +96,13 @@ double shell_key(int ox, int oy, int oz, double sx, double sy, double sz);
 uint64_t bits(double v);
 int64_t icbrt_floor(double x);
 
-// Pinned host staging for large downloads into caller memory: the results
-// are copied into the two buffers in turn while host threads move the
-// previous chunk into the caller's (pageable) memory.
+// Pinned host staging for downloads into caller memory: the device writes
+// into the two buffers in turn while host threads move the previous chunk
+// into the caller's (pageable) memory.
 struct Staging {
-  static constexpr size_t kBytes = size_t(64) << 20;  // per buffer
+  static constexpr size_t kBytes = size_t(64) << 20;  // per buffer, at most
   void* buf[2] = {nullptr, nullptr};
+  size_t cap[2] = {0, 0};
   hipEvent_t ev[2] = {nullptr, nullptr};
   std::mutex mu;
   Staging() = default;
@@ -237,7 +238,7 @@ struct tess_diagram {
   DevBuf<uint64_t> foff, fsums;
   DevBuf<tess_cell_stats> stats;
   DevBuf<SummarySlot> summary;  // kSummarySlots
-  DevBuf<uint32_t> work1, redo_list, redo_list2;
+  DevBuf<uint32_t> redo_list, redo_list2;
   // cells that exhausted the shell table / outgrew the largest LDS variant:
   // count at [0], grid positions from [1]
   DevBuf<uint32_t> tredo, spill;
@@ -311,12 +312,22 @@ struct tess_model {
 
 namespace tess {
 
-// dst <- src (device), bytes of it, ordered after the context stream's work
-// and finished on return.  Copies of 16 MiB or more go through the
-// context's pinned staging, chunk by chunk, overlapping the transfer of one
-// chunk with the host copy of the one before; smaller ones are one
-// hipMemcpy.
-hipError_t download(tess_ctx* c, void* dst, const void* src, size_t bytes);
+// dst <- src (device), bytes of it, for up to kCopyOutPieces arrays at once,
+// ordered after the context stream's work and finished on return.  The device
+// writes them into the context's pinned staging, chunk by chunk, the transfer
+// of one chunk overlapping the host copy of the one before.  Pieces without a
+// destination are passed over; sub (device): uint64 values minus *sub.
+struct Piece {
+  void* dst;
+  const void* src;
+  size_t bytes;
+  const uint64_t* sub = nullptr;
+};
+hipError_t download(tess_ctx* c, const Piece* pieces, int count);
+inline hipError_t download(tess_ctx* c, void* dst, const void* src, size_t bytes) {
+  const Piece p{dst, src, bytes};
+  return download(c, &p, 1);
+}
 // dst <- src, len bytes, on up to eight host threads in pieces of at least
 // 4 MiB (the staged download's copy out of pinned memory)
 void host_copy(char* dst, const char* src, size_t len);
