@@ -29,37 +29,7 @@ using namespace tess;
 namespace tess {
 
 // ---------------------------------------------------------------- shell table
-// Generation order of celery.rs:437-673: the centre, then offsets with three,
-// two (xy, xz, yz) and one (x, y, z) non-zero components, each block looping
-// over |o|-1 in lexicographic order with the sign patterns listed there.
-uint64_t generation_index(int64_t cpd, int ox, int oy, int oz) {
-  const uint64_t M = (uint64_t)(cpd - 1);
-  const uint64_t a = ox ? (uint64_t)std::abs(ox) - 1 : 0;
-  const uint64_t b = oy ? (uint64_t)std::abs(oy) - 1 : 0;
-  const uint64_t c = oz ? (uint64_t)std::abs(oz) - 1 : 0;
-  const uint64_t two = 1 + 8 * M * M * M, one = two + 12 * M * M;
-  if (!ox && !oy && !oz) return 0;
-  if (ox && oy && oz) {
-    static const int order[8] = {0, 1, 2, 4, 3, 5, 6, 7};
-    const int bits = ((ox < 0) << 2) | ((oy < 0) << 1) | (oz < 0);
-    return 1 + 8 * ((a * M + b) * M + c) + order[bits];
-  }
-  if (ox && oy) return two + 4 * (a * M + b) + (((ox < 0) << 1) | (oy < 0));
-  if (ox && oz) return two + 4 * M * M + 4 * (a * M + c) + (((ox < 0) << 1) | (oz < 0));
-  if (oy && oz) return two + 8 * M * M + 4 * (b * M + c) + (((oy < 0) << 1) | (oz < 0));
-  if (ox) return one + 2 * a + (ox < 0);
-  if (oy) return one + 2 * M + 2 * b + (oy < 0);
-  return one + 4 * M + 2 * c + (oz < 0);
-}
-
-// celery.rs:419-427: squared gap distance, (sq(gx sx) + sq(gy sy)) + sq(gz sz).
-double shell_key(int ox, int oy, int oz, double sx, double sy, double sz) {
-  if (!ox && !oy && !oz) return -1.0;
-  auto sq = [](double t) { return t * t; };
-  const double gx = ox ? std::abs(ox) - 1 : 0, gy = oy ? std::abs(oy) - 1 : 0,
-               gz = oz ? std::abs(oz) - 1 : 0;
-  return sq(gx * sx) + sq(gy * sy) + sq(gz * sz);
-}
+uint64_t generation_index(int64_t cpd, int ox, int oy, int oz) { return shell_generation(cpd, ox, oy, oz); }
 
 // Entries with |o|_inf <= L sorted by (key, generation index).  For L < cpd-1
 // only keys below kcut = min_a (L s_a)^2 are kept: every offset outside the
@@ -68,11 +38,7 @@ void build_table_host(int64_t cpd, double sx, double sy, double sz, int L, std::
                       std::vector<int32_t>& off, double* kcut) {
   if (L > cpd - 1) L = (int)(cpd - 1);
   const bool full = (L == cpd - 1);
-  double kc = std::numeric_limits<double>::infinity();
-  if (!full) {
-    auto sq = [](double t) { return t * t; };
-    kc = std::min(sq(L * sx), std::min(sq(L * sy), sq(L * sz)));
-  }
+  const double kc = table_kcut(cpd, sx, sy, sz, L);
   struct E {
     double k;
     uint64_t g;
@@ -95,6 +61,33 @@ void build_table_host(int64_t cpd, double sx, double sy, double sz, int L, std::
     off[t] = es[t].o;
   }
   *kcut = kc;
+}
+
+double table_kcut(int64_t cpd, double sx, double sy, double sz, int L) {
+  if (L >= cpd - 1) return std::numeric_limits<double>::infinity();
+  auto sq = [](double t) { return t * t; };
+  return std::min(sq(L * sx), std::min(sq(L * sy), sq(L * sz)));
+}
+
+// Entries per class of equal gaps: gap 0 of an axis holds o = -1, 0 and 1,
+// the others two offsets each.
+int table_len(int64_t cpd, double sx, double sy, double sz, int L) {
+  if (L <= 0) return 1;
+  const bool full = L >= cpd - 1;
+  const double kc = table_kcut(cpd, sx, sy, sz, L);
+  int len = 0;
+  for (int a = 0; a < L; ++a)
+    for (int b = 0; b < L; ++b)
+      for (int c = 0; c < L; ++c)
+        if (full || shell_gap_key(a, b, c, sx, sy, sz) < kc) len += (a ? 2 : 3) * (b ? 2 : 3) * (c ? 2 : 3);
+  // the centre (key -1) is counted with gap 0
+  if (!full && !(shell_gap_key(0, 0, 0, sx, sy, sz) < kc)) len += -1.0 < kc ? 1 : 0;
+  return len;
+}
+
+bool table_on_device(int64_t cpd, double sx, double sy, double sz, int L) {
+  return L <= kTableDeviceL && cpd >= 1 && std::isfinite(sx) && std::isfinite(sy) && std::isfinite(sz) && sx >= 0 &&
+         sy >= 0 && sz >= 0;
 }
 
 uint64_t bits(double v) {

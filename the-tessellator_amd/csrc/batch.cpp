@@ -37,12 +37,6 @@ using namespace tess;
 
 namespace {
 
-struct HostTable {
-  std::vector<double> key;
-  std::vector<int32_t> off;
-  double kcut = 0;
-};
-
 using TableKey = std::tuple<int64_t, uint64_t, uint64_t, uint64_t>;
 
 struct Graph {
@@ -94,13 +88,13 @@ struct tess_batch {
   DevBuf<CellArgs> args;
   DevBuf<double> tkey;
   DevBuf<int32_t> toff;
+  DevBuf<TableBuild> tbuild;
   // learned order
   DevBuf<uint16_t> feat;
   DevBuf<float> pred, cost;
   DevBuf<uint32_t> skey, shist, ssums, order;
   std::vector<std::unique_ptr<tess_diagram>> views;
   std::vector<GridDev> hgrid;
-  std::map<TableKey, std::shared_ptr<HostTable>> tables;
   std::vector<TableKey> table_of;  // per set, as uploaded
   Graph gbin, gcells;
   std::vector<int64_t> gcells_key;  // config + slot counts the cells graph was captured for
@@ -229,78 +223,74 @@ tess_status build_bin_graph(tess_batch* b) {
   return err != TESS_OK ? err : st;
 }
 
-// Shell tables for every set's grid (host, in parallel, cached by shape),
-// uploaded as one combined table, and the per-set kernel arguments.
+// Shell tables for every set's grid, built on the device as one combined
+// table, and the per-set kernel arguments.
 tess_status prepare_tables(tess_batch* b, double* table_ms) {
   tess_ctx* c = b->ctx;
   auto t0 = std::chrono::steady_clock::now();
   std::vector<TableKey> keys(b->nsets);
-  std::vector<TableKey> missing;
   for (size_t s = 0; s < b->nsets; ++s) {
     const GridDev& G = b->hgrid[s];
     keys[s] = std::make_tuple((int64_t)G.cpd, bits(G.sx), bits(G.sy), bits(G.sz));
-    if (!b->tables.count(keys[s])) {
-      b->tables[keys[s]] = nullptr;
-      missing.push_back(keys[s]);
-    }
-  }
-  if (!missing.empty()) {
-    std::vector<std::shared_ptr<HostTable>> built(missing.size());
-    const unsigned hw = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
-    std::vector<std::thread> pool;
-    for (unsigned t = 0; t < hw; ++t)
-      pool.emplace_back([&, t]() {
-        for (size_t i = t; i < missing.size(); i += hw) {
-          auto h = std::make_shared<HostTable>();
-          const TableKey& k = missing[i];
-          double sxv, syv, szv;
-          uint64_t u;
-          u = std::get<1>(k);
-          std::memcpy(&sxv, &u, 8);
-          u = std::get<2>(k);
-          std::memcpy(&syv, &u, 8);
-          u = std::get<3>(k);
-          std::memcpy(&szv, &u, 8);
-          build_table_host(std::get<0>(k), sxv, syv, szv, kTableL, h->key, h->off, &h->kcut);
-          built[i] = h;
-        }
-      });
-    for (auto& th : pool) th.join();
-    for (size_t i = 0; i < missing.size(); ++i) b->tables[missing[i]] = built[i];
   }
   if (keys != b->table_of) {
-    // combined upload and per-set arguments
     size_t total = 0;
-    std::vector<size_t> tb(b->nsets);
+    std::vector<TableBuild> tb(b->nsets);
+    std::vector<size_t> at(b->nsets);
+    std::vector<size_t> host;  // sets whose table the device does not build
     for (size_t s = 0; s < b->nsets; ++s) {
-      tb[s] = total;
-      total += b->tables[keys[s]]->key.size();
+      const GridDev& G = b->hgrid[s];
+      TableBuild& t = tb[s];
+      t.cpd = G.cpd;
+      t.sx = G.sx;
+      t.sy = G.sy;
+      t.sz = G.sz;
+      t.L = (int)std::min<int64_t>(kTableL, (int64_t)G.cpd - 1);
+      t.kcut = table_kcut(G.cpd, G.sx, G.sy, G.sz, t.L);
+      t.len = 0;
+      at[s] = total;
+      if (table_on_device(G.cpd, G.sx, G.sy, G.sz, t.L)) {
+        t.len = table_len(G.cpd, G.sx, G.sy, G.sz, t.L);
+        total += (size_t)t.len;
+      } else {
+        host.push_back(s);
+        total += (size_t)(2 * t.L + 1) * (2 * t.L + 1) * (2 * t.L + 1);
+      }
     }
-    std::vector<double> hk(total);
-    std::vector<int32_t> ho(total);
-    for (size_t s = 0; s < b->nsets; ++s) {
-      const HostTable& h = *b->tables[keys[s]];
-      std::copy(h.key.begin(), h.key.end(), hk.begin() + tb[s]);
-      std::copy(h.off.begin(), h.off.end(), ho.begin() + tb[s]);
-    }
-    if (b->tkey.alloc(total) != hipSuccess || b->toff.alloc(total) != hipSuccess)
+    if (b->tkey.alloc(total) != hipSuccess || b->toff.alloc(total) != hipSuccess ||
+        b->tbuild.alloc(b->nsets) != hipSuccess)
       return c->fail(TESS_E_NOMEM, "device allocation failed");
+    for (size_t s = 0; s < b->nsets; ++s) {
+      tb[s].key = b->tkey.p + at[s];
+      tb[s].off = b->toff.p + at[s];
+    }
+    tess_status st;
+    if ((st = c->hip(hipMemcpy(b->tbuild.p, tb.data(), sizeof(TableBuild) * b->nsets, hipMemcpyHostToDevice),
+                     "upload")) != TESS_OK ||
+        (st = c->hip(launch_table(b->tbuild.p, (int)b->nsets, TableBuild{}, c->stream), "shell tables")) != TESS_OK)
+      return st;
+    for (size_t s : host) {
+      TableBuild& t = tb[s];
+      std::vector<double> k;
+      std::vector<int32_t> o;
+      build_table_host(t.cpd, t.sx, t.sy, t.sz, t.L, k, o, &t.kcut);
+      t.len = (int)k.size();
+      if ((st = c->hip(hipMemcpy(t.key, k.data(), 8 * k.size(), hipMemcpyHostToDevice), "upload")) != TESS_OK ||
+          (st = c->hip(hipMemcpy(t.off, o.data(), 4 * o.size(), hipMemcpyHostToDevice), "upload")) != TESS_OK)
+        return st;
+    }
     std::vector<CellArgs> ha(b->nsets);
     for (size_t s = 0; s < b->nsets; ++s) {
-      const HostTable& h = *b->tables[keys[s]];
       Table t;
-      t.key.view(b->tkey.p + tb[s], h.key.size());
-      t.off.view(b->toff.p + tb[s], h.off.size());
-      t.len = (int)h.key.size();
-      t.kcut = h.kcut;
+      t.key.view(tb[s].key, (size_t)tb[s].len);
+      t.off.view(tb[s].off, (size_t)tb[s].len);
+      t.len = tb[s].len;
+      t.kcut = tb[s].kcut;
       t.L = kTableL;
       ha[s] = base_args(b->views[s].get(), &t);
       ha[s].defer_table = 1;  // the passes list them (BatchArgs::tredo)
     }
-    tess_status st;
-    if ((st = c->hip(hipMemcpy(b->tkey.p, hk.data(), 8 * total, hipMemcpyHostToDevice), "upload")) != TESS_OK ||
-        (st = c->hip(hipMemcpy(b->toff.p, ho.data(), 4 * total, hipMemcpyHostToDevice), "upload")) != TESS_OK ||
-        (st = c->hip(hipMemcpy(b->args.p, ha.data(), sizeof(CellArgs) * b->nsets, hipMemcpyHostToDevice),
+    if ((st = c->hip(hipMemcpy(b->args.p, ha.data(), sizeof(CellArgs) * b->nsets, hipMemcpyHostToDevice),
                      "upload")) != TESS_OK)
       return st;
     b->table_of = keys;

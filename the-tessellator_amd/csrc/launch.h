@@ -92,6 +92,19 @@ hipError_t launch_copy_out(const CopyOut& a, hipStream_t s);
 // out[k] = src[at[k]], k < n
 hipError_t launch_pick_u64(const uint64_t* src, const uint64_t* at, int n, uint64_t* out, hipStream_t s);
 
+// table.hip: the first len entries of the shell table of a grid shape (cpd
+// cells per dimension of sizes s), |o|_inf <= L, keys below kcut: as
+// build_table_host leaves them.  many: `count` of them (device), else `one`.
+constexpr int kTableDeviceL = 12;
+struct TableBuild {
+  int64_t cpd;
+  double sx, sy, sz, kcut;
+  double* key;
+  int32_t* off;
+  int32_t L, len;
+};
+hipError_t launch_table(const TableBuild* many, int count, const TableBuild& one, hipStream_t s);
+
 // cell.hip: vpl = vertex slots per lane (1, 2 or 4)
 hipError_t launch_cells(int vpl, const CellArgs& a, hipStream_t s);
 // the same cells staging their geometry (CellArgs::geo_*), with the cell

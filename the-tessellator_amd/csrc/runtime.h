@@ -88,11 +88,16 @@ struct Table {
 // (celery.rs:418-679), see build_table_host.
 void build_table_host(int64_t cpd, double sx, double sy, double sz, int L, std::vector<double>& key,
                       std::vector<int32_t>& off, double* kcut);
-constexpr int kTableL = 12;
-// Position of an offset in the generation loops of celery.rs:437-673, and its
-// key (sq(gx sx) + sq(gy sy)) + sq(gz sz) of the gaps (celery.rs:419-427).
+constexpr int kTableL = kTableDeviceL;
+// Position of an offset in the generation loops (shell_generation).
 uint64_t generation_index(int64_t cpd, int ox, int oy, int oz);
-double shell_key(int ox, int oy, int oz, double sx, double sy, double sz);
+// Its kcut and its length without building it (L at most cpd - 1), and
+// whether launch_table may build it: at most kTableDeviceL rings, finite cell
+// sizes that are not negative (a longer table's classes outgrow the kernel's
+// LDS, and its sort is a rerun's).
+double table_kcut(int64_t cpd, double sx, double sy, double sz, int L);
+int table_len(int64_t cpd, double sx, double sy, double sz, int L);
+bool table_on_device(int64_t cpd, double sx, double sy, double sz, int L);
 uint64_t bits(double v);
 int64_t icbrt_floor(double x);
 
@@ -151,11 +156,35 @@ struct tess_ctx {
     auto key = std::make_tuple(cpd, bits(sx), bits(sy), bits(sz), L);
     auto it = tables.find(key);
     if (it != tables.end()) return it->second.get();
+    auto t = std::make_unique<Table>();
+    if (table_on_device(cpd, sx, sy, sz, L)) {
+      TableBuild b;
+      b.cpd = cpd;
+      b.sx = sx;
+      b.sy = sy;
+      b.sz = sz;
+      b.L = (int)std::min<int64_t>(L, cpd - 1);
+      b.kcut = t->kcut = table_kcut(cpd, sx, sy, sz, b.L);
+      b.len = t->len = table_len(cpd, sx, sy, sz, b.L);
+      t->L = L;
+      if (t->key.alloc(b.len) != hipSuccess || t->off.alloc(b.len) != hipSuccess) {
+        *st = fail(TESS_E_NOMEM, "shell table allocation failed");
+        return nullptr;
+      }
+      b.key = t->key.p;
+      b.off = t->off.p;
+      if (launch_table(nullptr, 1, b, stream) != hipSuccess) {
+        *st = fail(TESS_E_DEVICE, "shell table failed");
+        return nullptr;
+      }
+      Table* r = t.get();
+      tables[key] = std::move(t);
+      return r;
+    }
     std::vector<double> k;
     std::vector<int32_t> o;
     double kc;
     build_table_host(cpd, sx, sy, sz, L, k, o, &kc);
-    auto t = std::make_unique<Table>();
     if (t->key.alloc(k.size()) != hipSuccess || t->off.alloc(o.size()) != hipSuccess) {
       *st = fail(TESS_E_NOMEM, "shell table allocation failed");
       return nullptr;

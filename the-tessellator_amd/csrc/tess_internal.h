@@ -26,6 +26,42 @@ __host__ __device__ inline void unpack_off(int32_t p, int& ox, int& oy, int& oz)
   oz = (p & 1023) - 512;
 }
 
+__host__ __device__ inline int iabs(int v) { return v < 0 ? -v : v; }
+
+// Generation order of celery.rs:437-673: the centre, then offsets with three,
+// two (xy, xz, yz) and one (x, y, z) non-zero components, each block looping
+// over |o|-1 in lexicographic order with the sign patterns listed there.
+__host__ __device__ inline uint64_t shell_generation(int64_t cpd, int ox, int oy, int oz) {
+  const uint64_t M = (uint64_t)(cpd - 1);
+  const uint64_t a = ox ? (uint64_t)iabs(ox) - 1 : 0;
+  const uint64_t b = oy ? (uint64_t)iabs(oy) - 1 : 0;
+  const uint64_t c = oz ? (uint64_t)iabs(oz) - 1 : 0;
+  const uint64_t two = 1 + 8 * M * M * M, one = two + 12 * M * M;
+  if (!ox && !oy && !oz) return 0;
+  if (ox && oy && oz) {
+    // sign patterns in the order 0, 1, 2, 4, 3, 5, 6, 7
+    const int bits = ((ox < 0) << 2) | ((oy < 0) << 1) | (oz < 0);
+    return 1 + 8 * ((a * M + b) * M + c) + (bits == 3 ? 4 : bits == 4 ? 3 : bits);
+  }
+  if (ox && oy) return two + 4 * (a * M + b) + (((ox < 0) << 1) | (oy < 0));
+  if (ox && oz) return two + 4 * M * M + 4 * (a * M + c) + (((ox < 0) << 1) | (oz < 0));
+  if (oy && oz) return two + 8 * M * M + 4 * (b * M + c) + (((oy < 0) << 1) | (oz < 0));
+  if (ox) return one + 2 * a + (ox < 0);
+  if (oy) return one + 2 * M + 2 * b + (oy < 0);
+  return one + 4 * M + 2 * c + (oz < 0);
+}
+
+// celery.rs:419-427: squared gap distance, (sq(gx sx) + sq(gy sy)) + sq(gz sz).
+__host__ __device__ inline double shell_gap_key(int ga, int gb, int gc, double sx, double sy, double sz) {
+  const double x = ga * sx, y = gb * sy, z = gc * sz;
+  return x * x + y * y + z * z;
+}
+// The key of an offset: its gaps' (|o| - 1, 0 for o = 0); the centre comes first.
+__host__ __device__ inline double shell_key(int ox, int oy, int oz, double sx, double sy, double sz) {
+  if (!ox && !oy && !oz) return -1.0;
+  return shell_gap_key(ox ? iabs(ox) - 1 : 0, oy ? iabs(oy) - 1 : 0, oz ? iabs(oz) - 1 : 0, sx, sy, sz);
+}
+
 // Launch-wide counters accumulated by the cell kernel (one atomic per cell).
 struct Summary {
   unsigned long long flops;          // algorithmic f64 ops of all cells
