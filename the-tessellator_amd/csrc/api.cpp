@@ -277,17 +277,14 @@ tess_status bin(tess_diagram* d) {
   hipStream_t s = c->stream;
   tess_status st;
   if ((st = bin_enqueue(d, s)) != TESS_OK) return st;
-  if ((st = c->hip(hipMemcpyAsync(&d->hgrid, d->grid.p, sizeof(GridDev), hipMemcpyDeviceToHost, s),
-                   "grid copy")) != TESS_OK)
-    return st;
   // every point must have landed in exactly one grid cell before any pass
   // dereferences the sorted indices
-  uint32_t total = 0;
-  if ((st = c->hip(hipMemcpyAsync(&total, d->delim.p + d->nbins, 4, hipMemcpyDeviceToHost, s), "grid copy")) !=
-          TESS_OK ||
-      (st = c->hip(hipStreamSynchronize(s), "binning")) != TESS_OK)
-    return st;
-  if (total != (uint32_t)d->n) return c->fail(TESS_E_DEVICE, "counting sort lost points");
+  ReportArgs r{};
+  r.grid = d->grid.p;
+  r.binned = d->delim.p + d->nbins;
+  if ((st = pass_report(c, r, "binning")) != TESS_OK) return st;
+  d->hgrid = c->mail->grid;
+  if (c->mail->binned != (uint32_t)d->n) return c->fail(TESS_E_DEVICE, "counting sort lost points");
   d->binned = true;
   d->inv_ready = false;
   return TESS_OK;
@@ -462,11 +459,8 @@ tess_status compute_cells(tess_diagram* d, const Planner* plan) {
     sch.count[pick_vpl(d) >> 1] = n;  // vpl 1, 2, 4 -> slot 0, 1, 2
   }
   (void)hipEventRecord(ev.e[2], s);
-  if ((st = c->hip(hipMemsetAsync(d->summary.p, 0, kSummarySlots * sizeof(SummarySlot), s), "memset")) != TESS_OK ||
-      (st = c->hip(launch_fill_u32(d->redo.p, 1, 0u, s), "fill")) != TESS_OK ||
-      (st = c->hip(launch_fill_u32(d->tredo.p, 1, 0u, s), "fill")) != TESS_OK ||
-      (st = c->hip(launch_fill_u32(d->spill.p, 1, 0u, s), "fill")) != TESS_OK ||
-      (st = c->hip(launch_fill_u32((uint32_t*)d->arena_next, 2 * kArenaWords, 0u, s), "fill")) != TESS_OK)
+  if ((st = c->hip(launch_pass_begin({d->redo.p, d->tredo.p, d->spill.p, d->arena_next, d->summary.p}, s),
+                   "pass counters")) != TESS_OK)
     return st;
   // the planner's long-search list first (capacity 256, a table sized from
   // the largest predicted radius), then the capacity lists, largest first
@@ -479,30 +473,42 @@ tess_status compute_cells(tess_diagram* d, const Planner* plan) {
   for (int slot = 2; slot >= 0; --slot)
     if (sch.count[slot] && (st = run_cells(d, t, kVpl[slot], sch.list[slot], sch.count[slot], true)) != TESS_OK)
       return st;
+  // the face offsets are scanned before the host knows whether cells are to
+  // be rerun (most sets have none; three short kernels otherwise)
+  ReportArgs ra{};
+  ra.redo = d->redo.p;
+  ra.tredo = d->tredo.p;
+  ra.spill = d->spill.p;
+  ra.total = d->foff.p + n;
+  ra.extra = (const uint64_t*)d->arena_next + (size_t)kArenaStride * (kArenaParts + 1);
+  ra.summary = d->summary.p;
+  auto offsets = [&]() -> tess_status {
+    (void)hipEventRecord(ev.e[3], s);
+    const tess_status e = c->hip(launch_face_offsets(d->fcount.p, n, d->foff.p, d->fsums.p, s), "face offsets");
+    return e != TESS_OK ? e : pass_report(c, ra, "cell kernel");
+  };
+  if ((st = offsets()) != TESS_OK) return st;
   // cells that outgrew their capacity: rerun with the largest variant; after
   // a 64-vertex whole-set pass, first at 128 vertices (nearly all of them
   // fit, and that variant keeps more wavefronts resident) and the rest at 256
-  uint32_t nredo = 0;
-  if ((st = c->hip(hipMemcpyAsync(&nredo, d->redo.p, 4, hipMemcpyDeviceToHost, s), "redo")) != TESS_OK ||
-      (st = c->hip(hipStreamSynchronize(s), "cell kernel")) != TESS_OK)
-    return st;
+  const uint32_t nredo = c->mail->nredo;
   if (nredo) {
     if (d->redo_list.alloc(nredo) != hipSuccess) return c->fail(TESS_E_NOMEM, "device allocation failed");
     if ((st = c->hip(hipMemcpyAsync(d->redo_list.p, d->redo.p + 1, 4ull * nredo, hipMemcpyDeviceToDevice, s),
                      "redo")) != TESS_OK)
       return st;
     if (!plan && !d->geo_stage && pick_vpl(d) == 1) {
-      uint32_t nredo2 = 0;
       if ((st = c->hip(launch_fill_u32(d->redo.p, 1, 0u, s), "fill")) != TESS_OK ||
           (st = run_cells(d, t, 2, d->redo_list.p, (int)nredo, true)) != TESS_OK ||
-          (st = c->hip(hipMemcpyAsync(&nredo2, d->redo.p, 4, hipMemcpyDeviceToHost, s), "redo")) != TESS_OK ||
-          (st = c->hip(hipStreamSynchronize(s), "cell kernel")) != TESS_OK)
+          (st = pass_report(c, ra, "cell kernel")) != TESS_OK)
         return st;
+      const uint32_t nredo2 = c->mail->nredo;
       if (nredo2) {
         if (d->redo_list2.alloc(nredo2) != hipSuccess) return c->fail(TESS_E_NOMEM, "device allocation failed");
         if ((st = c->hip(hipMemcpyAsync(d->redo_list2.p, d->redo.p + 1, 4ull * nredo2, hipMemcpyDeviceToDevice, s),
                          "redo")) != TESS_OK ||
-            (st = run_cells(d, t, 4, d->redo_list2.p, (int)nredo2, true)) != TESS_OK)
+            (st = run_cells(d, t, 4, d->redo_list2.p, (int)nredo2, true)) != TESS_OK ||
+            (st = pass_report(c, ra, "cell kernel")) != TESS_OK)
           return st;
       }
     } else {
@@ -510,22 +516,26 @@ tess_status compute_cells(tess_diagram* d, const Planner* plan) {
         g->nredo = nredo;
         if ((st = geo_staging_alloc(d, g->rerun, nredo, 4)) != TESS_OK) return st;
       }
-      if ((st = run_cells(d, t, 4, d->redo_list.p, (int)nredo, true)) != TESS_OK) return st;
+      if ((st = run_cells(d, t, 4, d->redo_list.p, (int)nredo, true)) != TESS_OK ||
+          (st = pass_report(c, ra, "cell kernel")) != TESS_OK)
+        return st;
     }
   }
   // cells past the shell table or the largest LDS capacity
-  std::vector<uint32_t> tab, spl;
-  if ((st = read_list(c, d->tredo.p, tab)) != TESS_OK || (st = read_list(c, d->spill.p, spl)) != TESS_OK) return st;
+  const uint32_t ntab = c->mail->ntab, nspill = c->mail->nspill;
   FinishCounts fin;
-  const int ntab = (int)tab.size();
-  if (!tab.empty() || !spl.empty()) {
+  if (ntab || nspill) {
+    std::vector<uint32_t> tab, spl;
+    if ((st = read_items(c, d->tredo.p, ntab, tab)) != TESS_OK ||
+        (st = read_items(c, d->spill.p, nspill, spl)) != TESS_OK)
+      return st;
     CellArgs a = base_args(d, t);
     if ((st = finish_cells(d, a, std::move(tab), std::move(spl), &fin, d->geo_stage)) != TESS_OK) return st;
   }
   // planned passes: a cell whose search outran its table was under-sized by
   // the prediction too (marked after its rerun wrote its status)
   if (plan && ntab &&
-      (st = c->hip(launch_mark_status(d->tredo.p + 1, ntab, d->sorted.p, d->status.p,
+      (st = c->hip(launch_mark_status(d->tredo.p + 1, (int)ntab, d->sorted.p, d->status.p,
                                       d->opts.collect_stats ? d->stats.p : nullptr, TESS_CELL_FALLBACK, s),
                    "mark")) != TESS_OK)
     return st;
@@ -534,16 +544,9 @@ tess_status compute_cells(tess_diagram* d, const Planner* plan) {
                                                TESS_CELL_RERUN | (plan ? TESS_CELL_FALLBACK : 0u), s),
                             "mark")) != TESS_OK)
     return st;
-  (void)hipEventRecord(ev.e[3], s);
-  if ((st = c->hip(launch_face_offsets(d->fcount.p, n, d->foff.p, d->fsums.p, s), "face offsets")) != TESS_OK)
-    return st;
-  uint64_t total = 0;
-  unsigned long long used = 0;
-  if ((st = c->hip(hipMemcpyAsync(&total, d->foff.p + n, 8, hipMemcpyDeviceToHost, s), "total")) != TESS_OK ||
-      (st = c->hip(hipMemcpyAsync(&used, d->arena_next + (size_t)kArenaStride * (kArenaParts + 1), 8, hipMemcpyDeviceToHost, s),
-                   "arena")) != TESS_OK ||
-      (st = c->hip(hipStreamSynchronize(s), "face offsets")) != TESS_OK)
-    return st;
+  if ((nredo || ntab || nspill) && (st = offsets()) != TESS_OK) return st;
+  const uint64_t total = c->mail->total, used = c->mail->extra;
+  const Summary sm2 = c->mail->sum;
   if (used) return c->fail(TESS_E_CAPACITY, "the face arena is full");
   if (d->nbr.alloc(total) != hipSuccess || d->area.alloc(total) != hipSuccess)
     return c->fail(TESS_E_NOMEM, "device allocation failed");
@@ -552,12 +555,7 @@ tess_status compute_cells(tess_diagram* d, const Planner* plan) {
                    "compact")) != TESS_OK)
     return st;
   (void)hipEventRecord(ev.e[4], s);
-  SummarySlot slots[kSummarySlots];
-  if ((st = c->hip(hipMemcpyAsync(slots, d->summary.p, sizeof(slots), hipMemcpyDeviceToHost, s), "summary")) !=
-          TESS_OK ||
-      (st = c->hip(hipStreamSynchronize(s), "compute")) != TESS_OK)
-    return st;
-  const Summary sm2 = summary_total(slots);
+  if ((st = c->hip(hipStreamSynchronize(s), "compute")) != TESS_OK) return st;
   d->tim.bin_ms = ev.ms(0, 1);
   d->tim.plan_ms = ev.ms(1, 2);
   d->tim.cells_ms = ev.ms(2, 3);
@@ -604,7 +602,10 @@ tess_status tess_ctx_create(int dev, tess_ctx** out) {
   if (!c) return TESS_E_NOMEM;
   c->device = dev;
   (void)noalloc_setup(dev);  // the scratch address of this device, once
-  if (hipStreamCreate(&c->stream) != hipSuccess) {
+  if (hipStreamCreate(&c->stream) != hipSuccess ||
+      hipHostMalloc((void**)&c->mail, sizeof(PassReport), hipHostMallocCoherent) != hipSuccess) {
+    if (c->stream) (void)hipStreamDestroy(c->stream);
+    c->mail = nullptr;
     delete c;
     return TESS_E_DEVICE;
   }
@@ -851,7 +852,6 @@ tess_status single_cell(tess_diagram* d, size_t index, const double* site, doubl
   tess_status st;
   if (!d->binned) {
     if ((st = bin(d)) != TESS_OK) return st;
-    if ((st = c->hip(hipStreamSynchronize(s), "binning")) != TESS_OK) return st;
   }
   if (!site && !d->inv_ready) {
     if (d->inv.alloc(d->n) != hipSuccess) return c->fail(TESS_E_NOMEM, "device allocation failed");

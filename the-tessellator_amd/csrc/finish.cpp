@@ -46,12 +46,22 @@ tess_status read_list(tess_ctx* c, const uint32_t* dev, std::vector<uint32_t>& v
   if ((st = c->hip(hipMemcpyAsync(&n, dev, 4, hipMemcpyDeviceToHost, c->stream), "download")) != TESS_OK ||
       (st = c->hip(hipStreamSynchronize(c->stream), "download")) != TESS_OK)
     return st;
+  return read_items(c, dev, n, v);
+}
+
+tess_status read_items(tess_ctx* c, const uint32_t* dev, uint32_t n, std::vector<uint32_t>& v) {
+  tess_status st;
   v.resize(n);
   if (!n) return TESS_OK;
   if ((st = c->hip(hipMemcpyAsync(v.data(), dev + 1, 4ull * n, hipMemcpyDeviceToHost, c->stream), "download")) !=
       TESS_OK)
     return st;
   return c->hip(hipStreamSynchronize(c->stream), "download");
+}
+
+tess_status pass_report(tess_ctx* c, const ReportArgs& a, const char* what) {
+  const tess_status st = c->hip(launch_pass_report(a, c->mail, c->stream), what);
+  return st != TESS_OK ? st : c->hip(hipStreamSynchronize(c->stream), what);
 }
 
 tess_status finish_cells(tess_diagram* d, const CellArgs& a0, std::vector<uint32_t> tab, std::vector<uint32_t> spl,

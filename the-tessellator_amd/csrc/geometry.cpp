@@ -46,13 +46,14 @@ tess_status finish_geometry(tess_diagram* d, const GeoStage& g, GeoEvents& ev, d
       (st = c->hip(launch_face_offsets(d->geo_count.p, (int)n, d->geo_voff.p, d->geo_sums.p, s), "scan")) !=
           TESS_OK ||
       (st = c->hip(launch_face_offsets(d->geo_count.p + n, (int)n, d->geo_rbase.p, d->geo_sums.p, s), "scan")) !=
-          TESS_OK ||
-      (st = c->hip(hipMemcpyAsync(&d->geo_nv, d->geo_voff.p + n, 8, hipMemcpyDeviceToHost, s), "download")) !=
-          TESS_OK ||
-      (st = c->hip(hipMemcpyAsync(&d->geo_nr, d->geo_rbase.p + n, 8, hipMemcpyDeviceToHost, s), "download")) !=
-          TESS_OK ||
-      (st = c->hip(hipStreamSynchronize(s), "geometry")) != TESS_OK)
+          TESS_OK)
     return st;
+  ReportArgs ra{};
+  ra.total = d->geo_voff.p + n;
+  ra.extra = d->geo_rbase.p + n;
+  if ((st = pass_report(c, ra, "geometry")) != TESS_OK) return st;
+  d->geo_nv = c->mail->total;
+  d->geo_nr = c->mail->extra;
   const uint64_t F = d->total_faces;
   if (d->geo_v.alloc(3 * d->geo_nv) != hipSuccess || d->geo_roff.alloc(F + 1) != hipSuccess ||
       d->geo_ring.alloc(d->geo_nr) != hipSuccess)
@@ -67,7 +68,7 @@ tess_status finish_geometry(tess_diagram* d, const GeoStage& g, GeoEvents& ev, d
   for (size_t k = 0; k < g.extra.size(); ++k)
     if ((st = compact(*g.extra[k], g.extra_items[k])) != TESS_OK) return st;
   if ((st = compact(first, n)) != TESS_OK || (nredo && (st = compact(rerun, nredo)) != TESS_OK) ||
-      (st = c->hip(hipMemcpyAsync(d->geo_roff.p + F, &d->geo_nr, 8, hipMemcpyHostToDevice, s), "upload")) !=
+      (st = c->hip(hipMemcpyAsync(d->geo_roff.p + F, d->geo_rbase.p + n, 8, hipMemcpyDeviceToDevice, s), "copy")) !=
           TESS_OK ||
       (st = c->hip(hipEventRecord(ev.e[2], s), "event")) != TESS_OK ||
       (st = c->hip(hipStreamSynchronize(s), "geometry")) != TESS_OK ||

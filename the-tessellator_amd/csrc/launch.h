@@ -72,6 +72,31 @@ hipError_t launch_compact(const uint32_t* fcount, const uint64_t* foff, int n, c
                           const uint64_t* fpos = nullptr);
 hipError_t launch_invert(const uint32_t* sorted, int n, uint32_t* inv, hipStream_t s);
 
+// pass.hip: the counters of a cell pass cleared in one launch (null ones are
+// passed over): list lengths, arena_next's kArenaWords, kSummarySlots slots.
+struct PassCounters {
+  uint32_t *redo, *tredo, *spill;
+  unsigned long long* arena;
+  SummarySlot* summary;
+};
+hipError_t launch_pass_begin(const PassCounters& a, hipStream_t s);
+// What the host reads between passes (pinned host memory; null sources give
+// zeros): list lengths, the points in the delimiters, two 64-bit words, the
+// summary slots' sum, the grid.
+struct ReportArgs {
+  const uint32_t *redo, *tredo, *spill, *binned;
+  const uint64_t *total, *extra;
+  const SummarySlot* summary;
+  const GridDev* grid;
+};
+struct PassReport {
+  uint32_t nredo, ntab, nspill, binned;
+  uint64_t total, extra;
+  Summary sum;
+  GridDev grid;
+};
+hipError_t launch_pass_report(const ReportArgs& a, PassReport* host, hipStream_t s);
+
 // copyout.hip: bytes [base, base + len) of the pieces laid end to end, each
 // from a multiple of 16 (start), into dst (pinned host memory, 16-byte
 // aligned; len bytes rounded up to 16 are written).  sub: every uint64 of the

@@ -85,11 +85,8 @@ tess_status tess_diagram_cells_at_particles(tess_diagram* d, const double* xyz, 
     return c->fail(TESS_E_NOMEM, "device allocation failed");
   Events ev;
   if ((st = c->hip(hipMemcpyAsync(T.sites.p, xyz, 24 * m, hipMemcpyHostToDevice, s), "upload")) != TESS_OK ||
-      (st = c->hip(hipMemsetAsync(T.summary.p, 0, kSummarySlots * sizeof(SummarySlot), s), "memset")) != TESS_OK ||
-      (st = c->hip(launch_fill_u32(T.redo.p, 1, 0u, s), "fill")) != TESS_OK ||
-      (st = c->hip(launch_fill_u32(T.tredo.p, 1, 0u, s), "fill")) != TESS_OK ||
-      (st = c->hip(launch_fill_u32(T.spill.p, 1, 0u, s), "fill")) != TESS_OK ||
-      (st = c->hip(launch_fill_u32((uint32_t*)T.arena.p, 2 * kArenaWords, 0u, s), "fill")) != TESS_OK ||
+      (st = c->hip(launch_pass_begin({T.redo.p, T.tredo.p, T.spill.p, T.arena.p, T.summary.p}, s),
+                   "pass counters")) != TESS_OK ||
       (st = c->hip(hipEventRecord(ev.e[0], s), "event")) != TESS_OK)
     return st;
   CellArgs a = base_args(d, t);
@@ -140,53 +137,66 @@ tess_status tess_diagram_cells_at_particles(tess_diagram* d, const double* xyz, 
   a.defer_table = 1;
   const CellArgs a0 = a;
   if ((st = c->hip(launch_cells(vpl, a, s), "cell kernel")) != TESS_OK) return st;
-  uint32_t nredo = 0;
-  if ((st = c->hip(hipMemcpyAsync(&nredo, T.redo.p, 4, hipMemcpyDeviceToHost, s), "redo")) != TESS_OK ||
-      (st = c->hip(hipStreamSynchronize(s), "cell kernel")) != TESS_OK)
-    return st;
-  if (nredo && vpl < 4) {  // sites that outgrew the first pass: the largest variant
-    if (T.redo_list.alloc(nredo) != hipSuccess) return c->fail(TESS_E_NOMEM, "device allocation failed");
-    a.work = T.redo_list.p;
-    a.nwork = (int)nredo;
+  ReportArgs ra{};
+  ra.redo = T.redo.p;
+  ra.tredo = T.tredo.p;
+  ra.spill = T.spill.p;
+  ra.total = p->foff.p + m;
+  ra.summary = T.summary.p;
+  auto offsets = [&]() -> tess_status {
+    tess_status e = c->hip(hipEventRecord(ev.e[1], s), "event");
+    if (e == TESS_OK) e = c->hip(launch_face_offsets(p->fcount.p, (int)m, p->foff.p, T.fsums.p, s), "face offsets");
+    return e != TESS_OK ? e : pass_report(c, ra, "cell kernel");
+  };
+  if ((st = offsets()) != TESS_OK) return st;
+  // sites that outgrew the first pass: at 128 vertices after 64 (as in
+  // compute_cells), the rest at 256
+  const uint32_t nredo = c->mail->nredo;
+  uint32_t nleft = nredo;
+  for (int v = vpl * 2; nleft && v <= 4; v *= 2) {
+    DevBuf<uint32_t>& list = v == vpl * 2 ? T.redo_list : T.redo_list2;
+    if (list.alloc(nleft) != hipSuccess) return c->fail(TESS_E_NOMEM, "device allocation failed");
+    a.work = list.p;
+    a.nwork = (int)nleft;
     a.xcd_chunk = 0;
-    a.redo = T.spill.p + 1;
-    a.nredo = T.spill.p;
-    if ((st = c->hip(hipMemcpyAsync(T.redo_list.p, T.redo.p + 1, 4ull * nredo, hipMemcpyDeviceToDevice, s),
-                     "redo")) != TESS_OK ||
-        (st = c->hip(launch_cells(4, a, s), "cell kernel")) != TESS_OK)
+    a.redo = (v < 4 ? T.redo.p : T.spill.p) + 1;
+    a.nredo = v < 4 ? T.redo.p : T.spill.p;
+    if ((st = c->hip(hipMemcpyAsync(list.p, T.redo.p + 1, 4ull * nleft, hipMemcpyDeviceToDevice, s), "redo")) !=
+            TESS_OK ||
+        (st = c->hip(launch_fill_u32(T.redo.p, 1, 0u, s), "fill")) != TESS_OK ||
+        (st = c->hip(launch_cells(v, a, s), "cell kernel")) != TESS_OK ||
+        (st = pass_report(c, ra, "cell kernel")) != TESS_OK)
       return st;
+    nleft = c->mail->nredo;
   }
   // sites past the shell table or capacity 256
-  std::vector<uint32_t> tab, spl;
-  if ((st = read_list(c, T.tredo.p, tab)) != TESS_OK || (st = read_list(c, T.spill.p, spl)) != TESS_OK) return st;
+  const uint32_t ntab = c->mail->ntab, nspill = c->mail->nspill;
   FinishCounts fin;
-  if ((!tab.empty() || !spl.empty()) &&
-      (st = finish_cells(d, a0, std::move(tab), std::move(spl), &fin)) != TESS_OK)
-    return st;
+  if (ntab || nspill) {
+    std::vector<uint32_t> tab, spl;
+    if ((st = read_items(c, T.tredo.p, ntab, tab)) != TESS_OK ||
+        (st = read_items(c, T.spill.p, nspill, spl)) != TESS_OK ||
+        (st = finish_cells(d, a0, std::move(tab), std::move(spl), &fin)) != TESS_OK)
+      return st;
+  }
   if (nredo && vpl < 4 &&
       (st = c->hip(launch_mark_status(T.redo_list.p, (int)nredo, nullptr, p->status.p, a.stats, TESS_CELL_RERUN, s),
                    "mark")) != TESS_OK)
     return st;
-  if ((st = c->hip(hipEventRecord(ev.e[1], s), "event")) != TESS_OK ||
-      (st = c->hip(launch_face_offsets(p->fcount.p, (int)m, p->foff.p, T.fsums.p, s), "face offsets")) != TESS_OK ||
-      (st = c->hip(hipMemcpyAsync(&p->total, p->foff.p + m, 8, hipMemcpyDeviceToHost, s), "total")) != TESS_OK ||
-      (st = c->hip(hipStreamSynchronize(s), "face offsets")) != TESS_OK)
-    return st;
+  if ((nredo || ntab || nspill) && (st = offsets()) != TESS_OK) return st;
+  p->total = c->mail->total;
+  const Summary sm2 = c->mail->sum;
   if (p->nbr.alloc(p->total) != hipSuccess || p->area.alloc(p->total) != hipSuccess)
     return c->fail(TESS_E_NOMEM, "device allocation failed");
-  SummarySlot slots[kSummarySlots];
   float ms[2] = {0, 0};
   if ((st = c->hip(launch_compact(p->fcount.p, p->foff.p, (int)m, T.snbr.p, T.sarea.p, p->nbr.p, p->area.p, s,
                                   T.fpos.p),
                    "compact")) != TESS_OK ||
       (st = c->hip(hipEventRecord(ev.e[2], s), "event")) != TESS_OK ||
-      (st = c->hip(hipMemcpyAsync(slots, T.summary.p, sizeof(slots), hipMemcpyDeviceToHost, s), "summary")) !=
-          TESS_OK ||
       (st = c->hip(hipStreamSynchronize(s), "compact")) != TESS_OK ||
       (st = c->hip(hipEventElapsedTime(&ms[0], ev.e[0], ev.e[1]), "event")) != TESS_OK ||
       (st = c->hip(hipEventElapsedTime(&ms[1], ev.e[1], ev.e[2]), "event")) != TESS_OK)
     return st;
-  const Summary sm2 = summary_total(slots);
   p->ms[0] = ms[0];
   p->ms[1] = ms[1];
   p->reruns = vpl < 4 ? nredo : 0;

@@ -153,6 +153,13 @@ tess_status query_impl(tess_diagram* d, int kind, const double* xyz, size_t nq, 
   a.tlen = t ? t->len : 0;
   a.count = cnt.p;
   Events ev;
+  auto read_total = [&](const uint64_t* p, uint64_t* out, const char* what) -> tess_status {
+    ReportArgs r{};
+    r.total = p;
+    const tess_status e = pass_report(c, r, what);
+    if (e == TESS_OK) *out = c->mail->total;
+    return e;
+  };
   // Filtered kinds (real radius, grouped clouds): the unfiltered walk gives
   // upper bounds from the delimiters alone, one fill pass writes the kept
   // ids into the bound slots and counts them, and a compaction packs them:
@@ -169,8 +176,7 @@ tess_status query_impl(tess_diagram* d, int kind, const double* xyz, size_t nq, 
         (st = c->hip(launch_query_count(b, s), "query bound")) != TESS_OK ||
         (st = c->hip(hipEventRecord(ev.e[1], s), "event")) != TESS_OK ||
         (st = c->hip(launch_face_offsets(cnt.p, (int)nq, boff.p, sums.p, s), "query scan")) != TESS_OK ||
-        (st = c->hip(hipMemcpyAsync(&bound, boff.p + nq, 8, hipMemcpyDeviceToHost, s), "download")) != TESS_OK ||
-        (st = c->hip(hipStreamSynchronize(s), "query bound")) != TESS_OK)
+        (st = read_total(boff.p + nq, &bound, "query bound")) != TESS_OK)
       return st;
     DevBuf<uint32_t>& slots = T.slots;
     if (bound <= kBoundMax && slots.alloc(bound) == hipSuccess) {
@@ -181,9 +187,7 @@ tess_status query_impl(tess_diagram* d, int kind, const double* xyz, size_t nq, 
           (st = c->hip(launch_query_fill(a, s), "query fill")) != TESS_OK ||
           (st = c->hip(hipEventRecord(ev.e[3], s), "event")) != TESS_OK ||
           (st = c->hip(launch_face_offsets(cnt.p, (int)nq, q->offsets.p, sums.p, s), "query scan")) != TESS_OK ||
-          (st = c->hip(hipMemcpyAsync(&q->total, q->offsets.p + nq, 8, hipMemcpyDeviceToHost, s), "download")) !=
-              TESS_OK ||
-          (st = c->hip(hipStreamSynchronize(s), "query fill")) != TESS_OK)
+          (st = read_total(q->offsets.p + nq, &q->total, "query fill")) != TESS_OK)
         return st;
       if (q->ids.alloc(q->total) != hipSuccess) return c->fail(TESS_E_NOMEM, "device allocation failed");
       float ms[3] = {0, 0, 0};
@@ -205,9 +209,7 @@ tess_status query_impl(tess_diagram* d, int kind, const double* xyz, size_t nq, 
       (st = c->hip(launch_query_count(a, s), "query count")) != TESS_OK ||
       (st = c->hip(hipEventRecord(ev.e[1], s), "event")) != TESS_OK ||
       (st = c->hip(launch_face_offsets(cnt.p, (int)nq, q->offsets.p, sums.p, s), "query scan")) != TESS_OK ||
-      (st = c->hip(hipMemcpyAsync(&q->total, q->offsets.p + nq, 8, hipMemcpyDeviceToHost, s), "download")) !=
-          TESS_OK ||
-      (st = c->hip(hipStreamSynchronize(s), "query count")) != TESS_OK)
+      (st = read_total(q->offsets.p + nq, &q->total, "query count")) != TESS_OK)
     return st;
   if (q->ids.alloc(q->total) != hipSuccess) return c->fail(TESS_E_NOMEM, "device allocation failed");
   a.offsets = q->offsets.p;

@@ -141,7 +141,11 @@ struct tess_ctx {
   DevBuf<uint32_t> fin_list, fin_ctr;
   DevBuf<uint32_t> fin_tab, fin_cap;
   DevBuf<uint64_t> fin_tab64, fin_cap64;
-  Staging stage;  // large downloads (tess::download)
+  Staging stage;  // downloads (tess::download)
+  PassReport* mail = nullptr;  // pinned; under mu
+  ~tess_ctx() {
+    if (mail) (void)hipHostFree(mail);
+  }
 
   tess_status fail(tess_status s, const std::string& m) {
     err = m;
@@ -305,7 +309,7 @@ struct tess_diagram {
     DevBuf<int32_t> snbr;
     DevBuf<uint64_t> fpos, fsums;
     DevBuf<unsigned long long> arena;
-    DevBuf<uint32_t> redo, redo_list, tredo, spill, keys, keys_out, iota, order;
+    DevBuf<uint32_t> redo, redo_list, redo_list2, tredo, spill, keys, keys_out, iota, order;
     DevBuf<uint8_t> sort_tmp;
     DevBuf<SummarySlot> summary;
   } stmp;
@@ -410,7 +414,11 @@ tess_status finish_cells(tess_diagram* d, const CellArgs& a, std::vector<uint32_
 // The no-allocation entry point's scratch address on `device` (noalloc.hip),
 // taken once per device with that device current.
 tess_status noalloc_setup(int device);
-// Reads a device list (count at [0], items from [1]) into v.
+// Reads a device list (count at [0], items from [1]) into v; with its length
+// known, the items alone.
 tess_status read_list(tess_ctx* c, const uint32_t* dev, std::vector<uint32_t>& v);
+tess_status read_items(tess_ctx* c, const uint32_t* dev, uint32_t n, std::vector<uint32_t>& v);
+// A report of the device's counters (c->mail), the stream's work finished.
+tess_status pass_report(tess_ctx* c, const ReportArgs& a, const char* what);
 
 }  // namespace tess
