@@ -455,6 +455,9 @@ tess_status tess_compute_noalloc(tess_ctx* ctx, const double* xyz_device, size_t
  * they are correctly rounded like the host's). */
 tess_status tess_diag_arith(tess_ctx* ctx, const double* a, const double* b, size_t n,
                             double* sqrt_a, double* recip_a, double* a_div_b);
+/* The sample order of epoch `pass` (from 0) of a training with `seed` and n
+ * samples. */
+tess_status tess_diag_shuffle(tess_ctx* ctx, uint64_t seed, uint64_t pass, uint32_t n, int32_t* out);
 
 #ifdef __cplusplus
 }

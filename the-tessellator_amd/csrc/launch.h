@@ -97,6 +97,14 @@ struct PassReport {
 };
 hipError_t launch_pass_report(const ReportArgs& a, PassReport* host, hipStream_t s);
 
+// shuffle.hip: p = Fisher and Yates's shuffle of 0 .. n - 1 by splitmix64 from
+// *state, which moves on past its n - 1 draws.  h, rank, cnt, list: n words,
+// first: n + 1, sums: ceil(n / 1024) + 1.
+struct ShuffleBufs {
+  uint32_t *h, *rank, *cnt, *first, *list, *sums;
+};
+hipError_t launch_shuffle(uint64_t* state, uint32_t n, const ShuffleBufs& b, int* p, hipStream_t s);
+
 // copyout.hip: bytes [base, base + len) of the pieces laid end to end, each
 // from a multiple of 16 (start), into dst (pinned host memory, 16-byte
 // aligned; len bytes rounded up to 16 are written).  sub: every uint64 of the
@@ -223,6 +231,10 @@ hipError_t launch_mlp_train_step(const uint16_t* X, const float* T, const int* i
                                  const uint16_t* W, const float* bias, float* grad, float* loss, hipStream_t s);
 hipError_t launch_targets(const tess_cell_stats* st, int n, double smin, float* T, uint16_t* vmax, hipStream_t s);
 hipError_t launch_grad_sum(const float* grad, int nslots, float* out, hipStream_t s);
+// Sums over n rows of two: out = sum T, sum (T - mean)^2 per column, added up
+// in a fixed tree in double; part: 4 kMomentBlocks doubles.
+constexpr int kMomentBlocks = 256;
+hipError_t launch_moments(const float* T, size_t n, double* part, double out[4], hipStream_t s);
 hipError_t launch_standardise(const float* T, size_t n, const float norm[4], float* Tn, hipStream_t s);
 // Predictions in length units and candidates: exp(norm[1] y0 + norm[0]) smin
 // and expm1(norm[3] y1 + norm[2]).

@@ -50,6 +50,15 @@ hipError_t grow(DevBuf<T>& b, size_t need, size_t keep, hipStream_t s) {
   return hipSuccess;
 }
 
+struct ShuffleSpace {
+  DevBuf<uint32_t> w;
+  bool alloc(size_t n, ShuffleBufs* b) {
+    if (w.alloc(5 * n + 1 + (n + 1023) / 1024 + 1) != hipSuccess) return false;
+    *b = {w.p, w.p + n, w.p + 2 * n, w.p + 3 * n, w.p + 4 * n + 1, w.p + 5 * n + 1};
+    return true;
+  }
+};
+
 tess_status refresh_weights(tess_model* m) {
   return m->ctx->hip(launch_weights_from_master(m->master.p, m->wbf.p, m->bias.p, m->ctx->stream), "weights");
 }
@@ -283,19 +292,14 @@ tess_status tess_model_train(tess_model* m, int epochs, int batch, float lr, uin
   hipStream_t s = c->stream;
   const size_t S = m->count;
   tess_status st;
-  // target statistics (host, double)
-  std::vector<float> T(2 * S);
-  if ((st = c->hip(hipMemcpy(T.data(), m->T.p, 4 * T.size(), hipMemcpyDeviceToHost), "download")) != TESS_OK)
-    return st;
-  double mean[2] = {0, 0}, var[2] = {0, 0};
-  for (size_t i = 0; i < S; ++i)
-    for (int k = 0; k < 2; ++k) mean[k] += T[2 * i + k];
-  for (int k = 0; k < 2; ++k) mean[k] /= (double)S;
-  for (size_t i = 0; i < S; ++i)
-    for (int k = 0; k < 2; ++k) var[k] += (T[2 * i + k] - mean[k]) * (T[2 * i + k] - mean[k]);
+  // target statistics (double)
+  DevBuf<double> part;
+  double mom[4];
+  if (part.alloc(4 * kMomentBlocks) != hipSuccess) return c->fail(TESS_E_NOMEM, "device allocation failed");
+  if ((st = c->hip(launch_moments(m->T.p, S, part.p, mom, s), "statistics")) != TESS_OK) return st;
   for (int k = 0; k < 2; ++k) {
-    const double sd = std::sqrt(var[k] / (double)S);
-    m->norm[2 * k] = (float)mean[k];
+    const double sd = std::sqrt(mom[2 + k] / (double)S);
+    m->norm[2 * k] = (float)(mom[k] / (double)S);
     m->norm[2 * k + 1] = (float)(sd > 1e-6 ? sd : 1.0);
   }
   DevBuf<float> Tn, grad, loss;
@@ -310,14 +314,13 @@ tess_status tess_model_train(tess_model* m, int epochs, int batch, float lr, uin
           TESS_OK ||
       (st = c->hip(launch_standardise(m->T.p, S, m->norm, Tn.p, s), "standardise")) != TESS_OK)
     return st;
-  std::vector<int> perm(S);
+  ShuffleSpace space;
+  ShuffleBufs sb;
+  if (!space.alloc(S, &sb)) return c->fail(TESS_E_NOMEM, "device allocation failed");
   std::vector<float> lh((size_t)nbatches * slots);
   uint64_t rs = seed;
   for (int ep = 0; ep < epochs; ++ep) {
-    std::iota(perm.begin(), perm.end(), 0);
-    for (size_t i = S - 1; i > 0; --i) std::swap(perm[i], perm[splitmix64(rs) % (i + 1)]);
-    if ((st = c->hip(hipMemcpyAsync(idx.p, perm.data(), 4 * S, hipMemcpyHostToDevice, s), "upload")) != TESS_OK)
-      return st;
+    if ((st = c->hip(launch_shuffle(&rs, (uint32_t)S, sb, idx.p, s), "shuffle")) != TESS_OK) return st;
     for (int b = 0; b < nbatches; ++b) {
       ++m->adam_steps;
       const float b1c = 1.f - std::pow(0.9f, (float)m->adam_steps);
@@ -506,6 +509,19 @@ tess_status tess_mlp_gradient(tess_model* m, const uint16_t* x, const float* t, 
     *loss = (float)(tot / (double)n);
   }
   return TESS_OK;
+}
+
+tess_status tess_diag_shuffle(tess_ctx* ctx, uint64_t seed, uint64_t pass, uint32_t n, int32_t* out) {
+  if (!ctx || !out || n == 0 || n > (uint32_t)INT32_MAX) return TESS_E_INVALID;
+  std::lock_guard<std::mutex> g(ctx->mu);
+  (void)hipSetDevice(ctx->device);
+  ShuffleSpace space;
+  ShuffleBufs sb;
+  DevBuf<int> p;
+  if (!space.alloc(n, &sb) || p.alloc(n) != hipSuccess) return ctx->fail(TESS_E_NOMEM, "device allocation failed");
+  uint64_t state = seed + pass * (uint64_t)(n - 1) * 0x9E3779B97F4A7C15ull;
+  tess_status st = ctx->hip(launch_shuffle(&state, n, sb, p.p, ctx->stream), "shuffle");
+  return st != TESS_OK ? st : ctx->hip(download(ctx, out, p.p, 4 * (size_t)n), "download");
 }
 
 tess_status tess_mfma_probe(tess_ctx* ctx, const uint16_t* a, const uint16_t* b, float* d) {

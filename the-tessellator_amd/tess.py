@@ -39,7 +39,7 @@ EXPORTS = [
     "tess_diagram_compute_scheduled", "tess_diagram_features", "tess_mlp_forward", "tess_mlp_gradient",
     "tess_mfma_probe", "tess_batch_create", "tess_batch_destroy", "tess_batch_sets", "tess_batch_set_config",
     "tess_batch_get_config", "tess_batch_compute", "tess_batch_tune", "tess_batch_total_faces",
-    "tess_batch_copy_cells", "tess_batch_timings", "tess_diag_arith", "tess_diagram_query",
+    "tess_batch_copy_cells", "tess_batch_timings", "tess_diag_arith", "tess_diag_shuffle", "tess_diagram_query",
     "tess_diagram_query_device", "tess_query_count", "tess_query_total", "tess_query_copy", "tess_query_device",
     "tess_query_timings", "tess_query_destroy", "tess_diagram_cells_at_particles", "tess_site_cells_count",
     "tess_site_cells_total_faces", "tess_site_cells_copy", "tess_site_cells_copy_stats", "tess_site_cells_timings",
@@ -160,6 +160,7 @@ def load_library(path: str | None = None) -> C.CDLL:
         "tess_batch_copy_cells": (C.c_int, [vp, sz, dp, dp, dp, dp, dp]),
         "tess_batch_timings": (C.c_int, [vp, C.POINTER(Timings)]),
         "tess_diag_arith": (C.c_int, [vp, dp, dp, sz, dp, dp, dp]),
+        "tess_diag_shuffle": (C.c_int, [vp, C.c_uint64, C.c_uint64, C.c_uint32, dp]),
         "tess_compute_noalloc": (C.c_int, [vp, vp, sz, dp, dp, C.c_double, vp, vp, vp, vp, vp, C.c_uint64,
                                            C.POINTER(C.c_uint64)]),
         "tess_diagram_query": (C.c_int, [vp, C.c_int, dp, sz, dp, sz, C.c_int64, C.POINTER(vp)]),
@@ -273,6 +274,11 @@ class Context:
         s, r, q = (np.empty_like(a) for _ in range(3))
         self.check(self.lib.tess_diag_arith(self.h, _ptr(a), _ptr(b), a.size, _ptr(s), _ptr(r), _ptr(q)))
         return s, r, q
+
+    def diag_shuffle(self, seed, epoch, n):
+        out = np.empty(n, np.int32)
+        self.check(self.lib.tess_diag_shuffle(self.h, seed, epoch, n, _ptr(out)))
+        return out
 
     def mfma_probe(self, a_bits, b_bits):
         """One 16x16x32 bf16 MFMA: a [16][32], b [32][16] bf16 bit patterns -> fp32 [16][16]."""
