@@ -178,3 +178,27 @@ def test_features_and_predictions(ctx, n, density):
     assert np.allclose(out, want, rtol=2.0**-22, atol=0)
     m.close()
     d.close()
+
+
+# the largest radius decides how long a shell table the clouds need: negative
+# ones alone, none, one past the default table, infinite and NaN ones, at the
+# first, a middle and the last place of one and of several workgroups' radii
+@pytest.mark.parametrize("nq", [2, 255, 1025, 5000])
+@pytest.mark.parametrize("odd", [None, 0.9, np.inf, np.nan, -np.inf])
+def test_cloud_radii_on_the_device(ctx, nq, odd):
+    rng = np.random.default_rng(nq)
+    pts, q = rng.random((6000, 3)), rng.random((nq, 3))
+    d = tess.Diagram(ctx, pts, np.zeros(3), np.ones(3), density=1.25)
+    d.compute()
+    for base in (0.01, -1.0):
+        for at in (0, nq // 2, nq - 1):
+            r = np.full(nq, base)
+            if odd is not None:
+                r[at] = odd
+            qt, rt = tess.DeviceArray(ctx, q), tess.DeviceArray(ctx, r)
+            res = d.query_device(tess.QUERY_CLOUD, qt.ptr, nq, rt.ptr, nq)
+            off, ids = res.copy()
+            ro, ri = orc.queries(tess.QUERY_CLOUD, pts, q, r, density=1.25)
+            assert np.array_equal(off, ro) and np.array_equal(ids, ri), (base, at)
+            res.close()
+    d.close()

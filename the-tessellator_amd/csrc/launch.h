@@ -202,6 +202,16 @@ hipError_t launch_fill_u32(uint32_t* p, size_t m, uint32_t v, hipStream_t s);
 // that launch_query_compact then packs)
 hipError_t launch_query_count(const QueryArgs& a, hipStream_t s);
 hipError_t launch_query_fill(const QueryArgs& a, hipStream_t s);
+// *key = the largest of m radii (+inf if any is NaN) as an integer of the
+// same order; radius_of_key gives it back.
+hipError_t launch_radius_max(const double* radius, size_t m, uint64_t* key, hipStream_t s);
+inline double radius_of_key(uint64_t key) {
+  const uint64_t sign = 1ull << 63, u = key & sign ? key ^ sign : ~key;
+  double r;
+  static_assert(sizeof(r) == sizeof(u), "64 bits");
+  __builtin_memcpy(&r, &u, 8);
+  return r;
+}
 hipError_t launch_query_compact(int nq, const uint64_t* from, const uint64_t* to, const uint32_t* src, uint32_t* dst,
                                 hipStream_t s);
 

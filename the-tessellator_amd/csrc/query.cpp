@@ -24,18 +24,24 @@ namespace {
 // whose cut-off min_a (L s_a)^2 exceeds every finite radius, so that the
 // entries with key <= radius are a prefix of the table; NaN and +inf radii
 // (no stop, celery.rs:1036) and large radii take the full order (L = cpd - 1).
-int cloud_table_extent(int64_t cpd, const GridDev& G, const double* r, size_t m) {
+int cloud_table_extent(int64_t cpd, const GridDev& G, double rmax) {
   const int full = (int)(cpd - 1);
-  double rmax = -std::numeric_limits<double>::infinity();
-  for (size_t i = 0; i < m; ++i) {
-    if (!(r[i] < std::numeric_limits<double>::infinity())) return full;
-    rmax = std::max(rmax, r[i]);
-  }
+  if (!(rmax < std::numeric_limits<double>::infinity())) return full;
   auto sq = [](double t) { return t * t; };
   auto kcut = [&](int L) { return std::min(sq(L * G.sx), std::min(sq(L * G.sy), sq(L * G.sz))); };
   int L = kTableL;
   while (L < full && !(kcut(L) > rmax)) L *= 2;
   return L < full ? L : full;
+}
+
+// The largest of m radii, +inf if any is NaN.
+double largest_radius(const double* r, size_t m) {
+  double rmax = -std::numeric_limits<double>::infinity();
+  for (size_t i = 0; i < m; ++i) {
+    if (!(r[i] < std::numeric_limits<double>::infinity())) return std::numeric_limits<double>::infinity();
+    rmax = std::max(rmax, r[i]);
+  }
+  return rmax;
 }
 
 // Query sets at least this large are taken in grid order.
@@ -87,16 +93,21 @@ tess_status query_impl(tess_diagram* d, int kind, const double* xyz, size_t nq, 
   const GridDev& G = d->hgrid;
   const Table* t = nullptr;
   if (kind == TESS_QUERY_CLOUD) {
-    // the table extent needs the radii on the host
-    std::vector<double> hr;
-    const double* r = radius;
+    // the table extent needs the largest radius on the host
+    double rmax = 0;
     if (device_inputs) {
-      hr.resize(nradius);
-      if ((st = c->hip(hipMemcpy(hr.data(), radius, 8 * nradius, hipMemcpyDeviceToHost), "download")) != TESS_OK)
+      DevBuf<uint64_t>& word = d->qtmp.rmax;
+      if (word.alloc(1) != hipSuccess) return c->fail(TESS_E_NOMEM, "device allocation failed");
+      ReportArgs ra{};
+      ra.total = word.p;
+      if ((st = c->hip(launch_radius_max(radius, nradius, word.p, s), "radii")) != TESS_OK ||
+          (st = pass_report(c, ra, "radii")) != TESS_OK)
         return st;
-      r = hr.data();
+      rmax = radius_of_key(c->mail->total);
+    } else {
+      rmax = largest_radius(radius, nradius);
     }
-    const int L = cloud_table_extent(d->cpd, G, r, nradius);
+    const int L = cloud_table_extent(d->cpd, G, rmax);
     if (L > 511) return c->fail(TESS_E_INVALID, "radius spans more than 511 grid cells");
     if (!(t = c->table(d->cpd, G.sx, G.sy, G.sz, L, &st))) return st;
   }

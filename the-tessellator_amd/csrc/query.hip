@@ -491,6 +491,45 @@ __global__ __launch_bounds__(256) void k_query_compact(int nq, const uint64_t* _
   }
 }
 
+namespace {
+
+// Largest radius, every workgroup's by one atomic on the order-keeping
+// integer.  A cloud query needs it on the host for its shell table; the radii
+// themselves took 200 us to come down and be looked through (200k of them).
+__global__ __launch_bounds__(256) void k_radius_max(const double* __restrict__ radius, size_t m,
+                                                    unsigned long long* __restrict__ key) {
+  __shared__ unsigned long long best[4];
+  unsigned long long b = 0;
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < m; i += (size_t)gridDim.x * 256) {
+    const double r = radius[i];
+    const unsigned long long u = (unsigned long long)__double_as_longlong(r == r ? r : (double)INFINITY);
+    const unsigned long long k = u >> 63 ? ~u : u | 1ull << 63;
+    b = k > b ? k : b;
+  }
+#pragma unroll
+  for (int o = 1; o < 64; o *= 2) {
+    const unsigned long long v = __shfl_xor(b, o);
+    b = v > b ? v : b;
+  }
+  if ((threadIdx.x & 63) == 0) best[threadIdx.x >> 6] = b;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 4; ++w) b = best[w] > b ? best[w] : b;
+    atomicMax(key, b);
+  }
+}
+
+}  // namespace
+
+hipError_t launch_radius_max(const double* radius, size_t m, uint64_t* key, hipStream_t s) {
+  hipError_t e = launch_fill_u32(reinterpret_cast<uint32_t*>(key), 2, 0u, s);
+  if (e != hipSuccess || m == 0) return e;
+  const size_t blocks = (m + 1023) / 1024;
+  hipLaunchKernelGGL(k_radius_max, dim3((unsigned)(blocks < 256 ? blocks : 256)), dim3(256), 0, s, radius, m,
+                     reinterpret_cast<unsigned long long*>(key));
+  return hipGetLastError();
+}
+
 hipError_t launch_query_count(const QueryArgs& a, hipStream_t s) { return launch_query_pass<false>(a, s); }
 hipError_t launch_query_fill(const QueryArgs& a, hipStream_t s) { return launch_query_pass<true>(a, s); }
 hipError_t launch_query_compact(int nq, const uint64_t* from, const uint64_t* to, const uint32_t* src, uint32_t* dst,

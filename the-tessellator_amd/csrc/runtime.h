@@ -297,7 +297,7 @@ struct tess_diagram {
   // grid order of large query sets, the kept ids' upper-bound slots
   struct {
     DevBuf<uint32_t> cnt, obins, ocnt, odelim, orank, oorder, osums, omisc, slots;
-    DevBuf<uint64_t> sums, boff;
+    DevBuf<uint64_t> sums, boff, rmax;
     DevBuf<double> ox, oy, oz;
   } qtmp;
   // temporaries of tess_diagram_cells_at_particles, kept between calls
