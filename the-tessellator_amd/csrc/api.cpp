@@ -245,7 +245,10 @@ tess_status alloc_all(tess_diagram* d) {
   return TESS_OK;
 }
 
-tess_status bin_enqueue(tess_diagram* d, hipStream_t s) {
+namespace {
+
+// Bounds, counting sort and gather of a set of any size.
+tess_status bin_general(tess_diagram* d, hipStream_t s) {
   tess_ctx* c = d->ctx;
   const int n = (int)d->n;
   const int nparts = (int)std::min<size_t>(256, (d->n + 255) / 256);
@@ -264,12 +267,28 @@ tess_status bin_enqueue(tess_diagram* d, hipStream_t s) {
   if ((st = c->hip(launch_counting_sort(d->x.p, d->y.p, d->z.p, n, d->grid.p, d->nbins, b, s, key), "sort")) !=
       TESS_OK)
     return st;
+  return c->hip(launch_gather(d->sorted.p, n, d->x.p, d->y.p, d->z.p, d->pts.p, s), "gather");
+}
+
+}  // namespace
+
+tess_status bin_enqueue(tess_diagram* d, hipStream_t s) {
+  tess_ctx* c = d->ctx;
+  const int n = (int)d->n;
+  tess_status st;
+  // small sets: one launch in the place of ten (k_bin_small)
+  const bool small = n <= kBinSmallPoints && d->nbins <= kBinSmallCells && d->opts.point_order == TESS_ORDER_INPUT;
+  if (small && (st = c->hip(launch_bin_small(d->x.p, d->y.p, d->z.p, n, (int)d->cpd, d->nbins, d->grid.p, d->bins.p,
+                                             d->delim.p, d->sorted.p, d->pts.p, s),
+                            "binning")) != TESS_OK)
+    return st;
+  if (!small && (st = bin_general(d, s)) != TESS_OK) return st;
   if (d->have_groups) {
     if (d->sgroups.alloc(d->n) != hipSuccess) return c->fail(TESS_E_NOMEM, "device allocation failed");
     if ((st = c->hip(launch_gather_groups(d->sorted.p, n, d->groups.p, d->sgroups.p, s), "gather")) != TESS_OK)
       return st;
   }
-  return c->hip(launch_gather(d->sorted.p, n, d->x.p, d->y.p, d->z.p, d->pts.p, s), "gather");
+  return TESS_OK;
 }
 
 tess_status bin(tess_diagram* d) {

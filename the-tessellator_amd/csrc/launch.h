@@ -23,6 +23,11 @@ struct SortBufs {
 hipError_t launch_counting_sort(const double* x, const double* y, const double* z, int n,
                                 const GridDev* g, int nbins, const SortBufs& b, hipStream_t s,
                                 const uint32_t* key = nullptr);
+// launch_bounds, launch_counting_sort (input order in a cell) and
+// launch_gather of a small set in one launch.
+constexpr int kBinSmallPoints = 12288, kBinSmallCells = 16384;
+hipError_t launch_bin_small(const double* x, const double* y, const double* z, int n, int cpd, int nbins, GridDev* g,
+                            uint32_t* bins, uint32_t* delim, uint32_t* sorted, PointRec* pts, hipStream_t s);
 // The counting sort of many point sets at once (a batch): set after set in
 // the SoA arrays, their grid cells numbered apart (set k's cells from
 // cbase[k]), their delimiters and sorted indices set-local, as
