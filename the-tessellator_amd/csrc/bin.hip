@@ -13,6 +13,7 @@
 //                canonical form of celery.rs:357-369), or ascending
 //                (Morton code, index) for the internal order
 //   k_gather     positions and ids in grid order (coalesced candidate loads)
+//   k_bin_small  all of it for a small set, in one workgroup
 //   k_compact    per-cell staged faces -> CSR
 // All passes are HBM-bound streams over the points or the cells.
 #include "launch.h"

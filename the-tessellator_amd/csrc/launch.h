@@ -201,7 +201,7 @@ hipError_t launch_mark_status(const uint32_t* list, int m, const uint32_t* sorte
                               tess_cell_stats* stats, uint32_t flag, hipStream_t s);
 hipError_t launch_fill_u32(uint32_t* p, size_t m, uint32_t v, hipStream_t s);
 
-// query.hip: radius queries, one wavefront per query (count, then fill at
+// query.hip: radius queries (count, then fill at
 // offsets from launch_face_offsets over the counts; a fill with count set
 // also writes the ids it kept per query, for fills into upper-bound slots
 // that launch_query_compact then packs)

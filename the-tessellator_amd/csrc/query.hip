@@ -9,8 +9,8 @@
 // cells of a row (i, j) that the radius reaches are one interval of k (the
 // gap distance only grows away from the query's cell), and consecutive cells
 // are consecutive in the grid order, so a row is one run of points (or cell
-// ids) found from two delimiters.  The count pass gives a query 16 lanes, a
-// row each; the fill pass one wavefront.  The neighbour cloud walks the shell
+// ids) found from two delimiters.  Both passes give a query 16 lanes, a row
+// each; long rows are walked by the whole wavefront.  The neighbour cloud walks the shell
 // table in canonical order, 64 entries per step, until the first key above
 // the radius.
 //
