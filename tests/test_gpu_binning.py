@@ -46,3 +46,22 @@ def test_small_sets(ctx, n, kind, density):
                          groups=np.arange(len(pts)) % 5, target_group=2)
     assert np.array_equal(off, ro) and np.array_equal(ids, ri)
     d.close()
+
+
+# sets of up to 1 MiB (43,690 points) reach the device through one pinned
+# buffer, one after the other: none may see the next one's points, and the
+# caller's array is free once the call is back
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 43690, 43691])
+def test_uploads_in_turn(ctx, n):
+    sets = [np.random.default_rng(k).random((n, 3)) for k in range(6)]
+    ds = []
+    for p in sets:
+        q = p.copy()
+        ds.append(tess.Diagram(ctx, q, np.full(3, -0.1), np.full(3, 1.1), density=2.0))
+        q[:] = 0.5
+    for p, d in zip(sets, ds):
+        d.query(tess.QUERY_CELLS, [[0.5, 0.5, 0.5]], 0.01)
+        _, bins, srt, dl = orc.grid(p, 2.0)
+        cell, sorted_, delim = d.copy_grid()
+        assert np.array_equal(cell, bins) and np.array_equal(sorted_, srt) and np.array_equal(delim, dl)
+        d.close()

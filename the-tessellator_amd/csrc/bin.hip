@@ -43,6 +43,19 @@ __global__ void k_soa(const double* __restrict__ xyz, int n, double* __restrict_
   z[i] = xyz[3 * (size_t)i + 2];
 }
 
+// From pinned host memory: every 16 bytes cross the link once, in order.
+__global__ __launch_bounds__(256) void k_soa_host(const double2* __restrict__ xyz, int n, double* __restrict__ x,
+                                                  double* __restrict__ y, double* __restrict__ z) {
+  const uint32_t c = blockIdx.x * 256 + threadIdx.x, m = 3u * (uint32_t)n;
+  if (2 * c >= m) return;
+  const double2 v = xyz[c];  // (the buffer is a whole number of 16 bytes)
+#pragma unroll
+  for (uint32_t k = 0; k < 2; ++k) {
+    const uint32_t i = 2 * c + k, p = i / 3, a = i - 3 * p;
+    if (i < m) (a == 0 ? x : a == 1 ? y : z)[p] = k ? v.y : v.x;
+  }
+}
+
 // Cell sizes as celery.rs:164-170: (max-min)/cpd and cpd/(max-min).
 __device__ __forceinline__ GridDev grid_of(const double lo[3], const double hi[3], int cpd) {
   const double c = (double)cpd;
@@ -706,6 +719,12 @@ inline int blocks(long long n, int t) { return (int)((n + t - 1) / t); }
 
 hipError_t launch_soa(const double* xyz, int n, double* x, double* y, double* z, hipStream_t s) {
   hipLaunchKernelGGL(k_soa, dim3(blocks(n, 256)), dim3(256), 0, s, xyz, n, x, y, z);
+  return hipGetLastError();
+}
+
+hipError_t launch_soa_host(const double* xyz, int n, double* x, double* y, double* z, hipStream_t s) {
+  hipLaunchKernelGGL(k_soa_host, dim3(blocks((3ll * n + 1) / 2, 256)), dim3(256), 0, s,
+                     reinterpret_cast<const double2*>(xyz), n, x, y, z);
   return hipGetLastError();
 }
 

@@ -6,6 +6,8 @@ namespace tess {
 
 // bin.hip
 hipError_t launch_soa(const double* xyz, int n, double* x, double* y, double* z, hipStream_t s);
+// the same from pinned host memory (16-byte aligned, read in 16 bytes a lane)
+hipError_t launch_soa_host(const double* xyz, int n, double* x, double* y, double* z, hipStream_t s);
 hipError_t launch_bounds(const double* x, const double* y, const double* z, int n, int cpd,
                          double* part, int nparts, GridDev* g, hipStream_t s);
 // counting sort: bins/cnt/delim/sorted/scratch sized by the caller

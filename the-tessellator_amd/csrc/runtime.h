@@ -143,8 +143,16 @@ struct tess_ctx {
   DevBuf<uint64_t> fin_tab64, fin_cap64;
   Staging stage;  // downloads (tess::download)
   PassReport* mail = nullptr;  // pinned; under mu
+  // Points of small sets on their way to the device: pinned, with the event
+  // after the kernel that reads them; under mu.
+  static constexpr size_t kUpBytes = size_t(1) << 20;
+  void* up = nullptr;
+  hipEvent_t up_ev = nullptr;
+  bool up_busy = false;
   ~tess_ctx() {
     if (mail) (void)hipHostFree(mail);
+    if (up) (void)hipHostFree(up);
+    if (up_ev) (void)hipEventDestroy(up_ev);
   }
 
   tess_status fail(tess_status s, const std::string& m) {
