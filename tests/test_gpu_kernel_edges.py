@@ -202,3 +202,21 @@ def test_cloud_radii_on_the_device(ctx, nq, odd):
             assert np.array_equal(off, ro) and np.array_equal(ids, ri), (base, at)
             res.close()
     d.close()
+
+
+# clouds are counted by 16 lanes each from 16,384 queries on; radii from none
+# to the whole table's, mixed within a wavefront
+@pytest.mark.parametrize("nq", [16383, 16384, 16385, 20001])
+@pytest.mark.parametrize("grouped", [False, True])
+def test_many_clouds(ctx, nq, grouped):
+    rng = np.random.default_rng(nq)
+    pts, q = rng.random((3000, 3)), rng.random((nq, 3)) * 1.2 - 0.1
+    groups = (np.arange(len(pts)) % 3).astype(np.int64)
+    r = rng.choice([-1.0, 0.0, 1e-300, 0.005, 0.01, 0.02], nq)
+    r[:: nq // 7] = 0.6
+    d = tess.Diagram(ctx, pts, np.full(3, -0.5), np.full(3, 1.5), density=1.25, groups=groups)
+    d.compute()
+    off, ids = d.query(tess.QUERY_CLOUD, q, r, target_group=1 if grouped else None)[:2]
+    ro, ri = orc.queries(tess.QUERY_CLOUD, pts, q, r, density=1.25, groups=groups, target_group=1 if grouped else -1)
+    assert np.array_equal(off, ro) and np.array_equal(ids, ri)
+    d.close()
