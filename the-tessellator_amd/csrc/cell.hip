@@ -349,7 +349,7 @@ struct Lds {
   __device__ __forceinline__ void set_next(int h, int n) { reinterpret_cast<uint16_t*>(rec)[2 * h + 1] = (uint16_t)n; }
 };
 
-enum { CUT_OK = 0, CUT_CAPACITY = 1, CUT_DEGENERATE = 2, CUT_GENERAL = 3 };
+enum { CUT_OK = 0, CUT_CAPACITY = 1, CUT_DEGENERATE = 2, CUT_GENERAL = 3, CUT_WIDE = 4 };
 
 template <int VPL, int PPL, int FPL>
 struct CellState {
@@ -814,13 +814,19 @@ __device__ __forceinline__ uint64_t mask_at(uint64_t reversed, uint32_t t) {
 // instead.  A face dies when it loses a pair and is not crossed: dead pairs
 // mark their faces, crossings unmark theirs.  INC: vertices on the plane.
 // *beyond: a new vertex has |v|^2 > r2.
+// TWO false: the form of nearly every cut, for at most 64 pairs before and
+// after it and no vertex on the plane, so that nothing of the second pair
+// register or of the plane's vertices is computed or asked for; CUT_WIDE, with
+// nothing written, when the cut needs a pair slot past 63 (or has no room).
+// 1M uniform cells 17.5 -> 16.3 ms, 2M clustered 55.2 -> 52.5, 256k FCC lattice
+// 4.33 -> 4.0, with the checks for room as one.
 // Measured with the rest of the cut path rewritten to the same ends (scalar
 // bookkeeping per cut instead of per test, arguments reloaded instead of
 // spilled): 20.7k instructions per uniform cell instead of 27.9k, no spilled
 // vector registers; cell pass of 1M uniform points 23.4 -> 18.3 ms, of 2M
-// clustered 73.5 -> 58.7 ms, of a 256k FCC lattice 5.8 -> 4.6 ms.  Left as
-// it is: VALU 75 % and scalar unit 69 % busy.
-template <int PPL>
+// clustered 73.5 -> 58.7 ms, of a 256k FCC lattice 5.8 -> 4.6 ms.  Bound by
+// issue: VALU 75 % and scalar unit 69 % busy.
+template <bool TWO, int PPL>
 __device__ __forceinline__ int clip_fast64(Lds<1, PPL, 1>& S, CellState<1, PPL, 1>& C, const uint64_t OM,
                                            const uint64_t INC, double pnx, double pny, double pnz, double off,
                                            int32_t tag, int seq, int lane, double r2, int* newv, bool* beyond) {
@@ -830,26 +836,29 @@ __device__ __forceinline__ int clip_fast64(Lds<1, PPL, 1>& S, CellState<1, PPL, 
   const uint2 w0 = C.w[0], w1 = C.w[1];
   const uint64_t a0 = mask_at(RO, w0.x), b0 = mask_at(RO, w0.y);
   uint64_t a1 = 0, b1 = 0;
-  if (C.PA[1]) {
+  if constexpr (TWO) {
     a1 = mask_at(RO, w1.x);
     b1 = mask_at(RO, w1.y);
   }
-  if (INC) {  // an Outside vertex next to one on the plane: the general clip's
+  if (TWO && INC) {  // an Outside vertex next to one on the plane: the general clip's
     const uint64_t RI = __brevll(INC);
     uint64_t slow = C.PA[0] & ((a0 & mask_at(RI, w0.y)) | (b0 & mask_at(RI, w0.x)));
-    if (C.PA[1]) slow |= C.PA[1] & ((a1 & mask_at(RI, w1.y)) | (b1 & mask_at(RI, w1.x)));
+    slow |= C.PA[1] & ((a1 & mask_at(RI, w1.y)) | (b1 & mask_at(RI, w1.x)));
     if (slow) return CUT_GENERAL;
   }
-  const uint64_t CM0 = C.PA[0] & (a0 ^ b0), CM1 = C.PA[1] & (a1 ^ b1);
-  const uint64_t PD0 = C.PA[0] & a0 & b0, PD1 = C.PA[1] & a1 & b1;
+  const uint64_t CM0 = C.PA[0] & (a0 ^ b0), CM1 = TWO ? C.PA[1] & (a1 ^ b1) : 0ull;
+  const uint64_t PD0 = C.PA[0] & a0 & b0, PD1 = TWO ? C.PA[1] & a1 & b1 : 0ull;
   const int n0 = popc(CM0), ncross = n0 + popc(CM1);
-  if (ncross < 3) return CUT_GENERAL;
   // 2. free slots: vertices (an Outside one is free: the cut removes it),
   //    pairs (dying ones are free), the new face
   const uint64_t vfree = ~C.VA[0] | OM;
-  const uint64_t pf0 = ~C.PA[0] | PD0, pf1 = ~C.PA[1] | PD1;
+  const uint64_t pf0 = ~C.PA[0] | PD0, pf1 = TWO ? ~C.PA[1] | PD1 : ~0ull;
   const int np0 = popc(pf0);
-  if (ncross > 64 || ncross > popc(vfree) || ncross > np0 + popc(pf1) || ~C.FA[0] == 0) return CUT_CAPACITY;
+  const int nvf = popc(vfree), npf = TWO ? np0 + popc(pf1) : np0;
+  int room = nvf < npf ? nvf : npf;  // (at most 64)
+  room = ~C.FA[0] ? room : 0;
+  if (ncross < 3) return CUT_GENERAL;
+  if (ncross > room) return TWO ? CUT_CAPACITY : CUT_WIDE;
   const int nf = ctz64(~C.FA[0]);
   // 3. free pair slot k to lane k.  Lanes with nothing to push write lane
   //    63, which is not read unless 64 lanes push (then none has nothing); a
@@ -857,7 +866,7 @@ __device__ __forceinline__ int clip_fast64(Lds<1, PPL, 1>& S, CellState<1, PPL, 
   const int kc = mbcnt(CM0, lane), kp = mbcnt(pf0, lane), kv = mbcnt(vfree, lane);
   int ps = push_lane(lane_bit(pf0) ? kp : 63, lane);
   uint64_t pnew0 = ballot(kp < ncross) & pf0, pnew1 = 0;
-  if (np0 < ncross) {
+  if (TWO && np0 < ncross) {
     const int k1 = np0 + mbcnt(pf1, lane);
     const int p1 = push_lane(lane_bit(pf1) && k1 < 64 ? k1 : (np0 ? 0 : 63), lane + 64);
     ps = lane < np0 ? ps : p1;
@@ -882,7 +891,7 @@ __device__ __forceinline__ int clip_fast64(Lds<1, PPL, 1>& S, CellState<1, PPL, 
   uint32_t hin, rin, rout, sv, br;
   uint64_t jobs;  // lanes with a crossing
   int k;          // which one
-  if (CM1 == 0) {
+  if (!TWO || CM1 == 0) {
     const int slots = pull_lane(kc, push_lane(lane_bit(vfree) ? kv : 63, lane) | (ps << 8));
     const bool o0 = lane_bit(a0);
     hin = (uint32_t)(2 * lane + (o0 ? 0 : 1));
@@ -1081,7 +1090,10 @@ __device__ __forceinline__ uint32_t cell_body(const CellArgs& args, const int gp
     C.FA[0] = 0x3full;
   }
   wave_sync();
-  if constexpr (VPL == 1) load_pairs(S, C, lane);
+  if constexpr (VPL == 1) {
+    load_pairs(S, C, lane);
+    C.w[1] = make_uint2(0, 0);  // read, masked off, while no second pair is live
+  }
   uint64_t r2_at[VPL];  // the vertex that attains r2
   double r2 = cell_r2_at(C, lane, r2_at);
 
@@ -1362,7 +1374,13 @@ __device__ __forceinline__ uint32_t cell_body(const CellArgs& args, const int gp
         bool beyond = false;  // a new vertex is farther out than r2
         if constexpr (VPL == 1) {
           const uint64_t INC = kept[0] & ~ballot(dv[0] - coff < -kTol);
-          rc = clip_fast64(S, C, OM[0], INC, cnx, cny, cnz, coff, ctag, 6 + (int)ncuts, lane, r2, &newv, &beyond);
+          rc = CUT_WIDE;
+          if (!C.PA[1] && !INC)
+            rc = clip_fast64<false>(S, C, OM[0], INC, cnx, cny, cnz, coff, ctag, 6 + (int)ncuts, lane, r2, &newv,
+                                    &beyond);
+          if (rc == CUT_WIDE)
+            rc = clip_fast64<true>(S, C, OM[0], INC, cnx, cny, cnz, coff, ctag, 6 + (int)ncuts, lane, r2, &newv,
+                                   &beyond);
         } else {
           classify();
           rc = clip_fast(S, C, OM, cnx, cny, cnz, coff, ctag, 6 + (int)ncuts, lane, &newv);
