@@ -1027,9 +1027,10 @@ __device__ __forceinline__ const CellArgs& again(const CellArgs& A) {
 // One cell: the site at grid position gpos of the set A.  Returns the
 // cell's status bits (wave-uniform); the caller queues capacity reruns.
 // GEO: 0 the cell outputs, 1 the staged geometry only, 2 both.
-// WIN: stream slices per chunk (2 for the plain launch, 4 for the batched
-// one).
-template <int VPL, int PPL, int FPL, int GEO = 0, int WIN = 2>
+// WIN: stream slices per chunk (3 for the plain launch, 4 for the batched
+// one; plain, 2M clustered points: 52.4 ms at 2, 51.5 at 3, 51.8 at 4; 1M
+// uniform 16.3, 16.3, 16.4).
+template <int VPL, int PPL, int FPL, int GEO = 0, int WIN = 3>
 __device__ __forceinline__ uint32_t cell_body(const CellArgs& args, const int gpos, Lds<VPL, PPL, FPL>& S,
                                               const int lane, const int slot = 0) {
   using L = Lds<VPL, PPL, FPL>;
