@@ -1027,9 +1027,9 @@ __device__ __forceinline__ const CellArgs& again(const CellArgs& A) {
 // One cell: the site at grid position gpos of the set A.  Returns the
 // cell's status bits (wave-uniform); the caller queues capacity reruns.
 // GEO: 0 the cell outputs, 1 the staged geometry only, 2 both.
-// WIN: stream slices per chunk (3 for the plain launch, 4 for the batched
-// one; plain, 2M clustered points: 52.4 ms at 2, 51.5 at 3, 51.8 at 4; 1M
-// uniform 16.3, 16.3, 16.4).
+// WIN: stream slices per chunk.  Plain, 2M clustered points: 52.4 ms at 2,
+// 51.5 at 3, 51.8 at 4; 1M uniform 16.3, 16.3, 16.4; batched, 24 uniform sets:
+// 37.6 ms at 2 and 3, 37.9 at 4, 2M clustered 52.6, 51.5, 51.8.
 template <int VPL, int PPL, int FPL, int GEO = 0, int WIN = 3>
 __device__ __forceinline__ uint32_t cell_body(const CellArgs& args, const int gpos, Lds<VPL, PPL, FPL>& S,
                                               const int lane, const int slot = 0) {
@@ -1753,7 +1753,7 @@ template <int VPL, int PPL, int FPL>
 __device__ __forceinline__ void batch_item(const BatchArgs& B, uint64_t it, Lds<VPL, PPL, FPL>& S, int lane) {
   ConstArgs* cs = (ConstArgs*)(B.sets) + (uint32_t)uni_i((int)(it >> 32));
   const CellArgs& A = *(const CellArgs*)cs;
-  const uint32_t status = cell_body<VPL, PPL, FPL, 0, 4>(A, uni_i((int)(uint32_t)it), S, lane);
+  const uint32_t status = cell_body<VPL, PPL, FPL>(A, uni_i((int)(uint32_t)it), S, lane);
   if (lane == 0 && (status & TESS_CELL_CAPACITY) && B.redo) {
     const uint32_t slot = atomicAdd(B.nredo, 1u);
     B.redo[slot] = it;
