@@ -200,6 +200,12 @@ struct QueryBox {
   double r2;
 };
 
+// A z extent past the largest double has cells of infinite size: a gap of 0
+// cells is then no number (0 x inf) and out of reach, a gap of 1 and more in
+// reach of an infinite radius^2, and a row's cells in reach are no interval.
+// Its rows are taken cell by cell.
+__device__ __forceinline__ bool cell_by_cell(const GridDev& G) { return !(G.sz < (double)INFINITY); }
+
 __device__ __forceinline__ QueryBox query_box(const GridDev& G, double qx, double qy, double qz, double r) {
   QueryBox q;
   const int cpd = G.cpd;
@@ -217,6 +223,7 @@ __device__ __forceinline__ QueryBox query_box(const GridDev& G, double qx, doubl
   q.nj = nj > 0 ? (uint32_t)nj : 0u;
   // a NaN radius admits no cell (ds <= NaN is false): skip the walk
   q.rows = ni > 0 && nj > 0 && q.k1 >= q.k0 && r == r ? (uint32_t)ni * (uint32_t)nj : 0u;
+  if (cell_by_cell(G)) q.rows *= (uint32_t)(q.k1 - q.k0 + 1);  // (at most cpd^3, 10^9)
   return q;
 }
 
@@ -229,6 +236,12 @@ __device__ __forceinline__ QueryBox query_box(const GridDev& G, double qx, doubl
 // bounded on the other side by the box.
 __device__ __forceinline__ uint32_t query_row(const GridDev& G, const QueryBox& q, uint32_t t, uint32_t& first) {
   const int cpd = G.cpd;
+  int k = 0;
+  if (cell_by_cell(G)) {
+    const uint32_t nk = (uint32_t)(q.k1 - q.k0 + 1);
+    k = q.k0 + (int)(t % nk);
+    t /= nk;
+  }
   const int i = q.i0 + (int)(t / q.nj), j = q.j0 + (int)(t % q.nj);
   const double gx = (double)cell_gap(q.hx, i) * G.sx, gy = (double)cell_gap(q.hy, j) * G.sy;
   const double g2 = gx * gx + gy * gy;
@@ -237,6 +250,10 @@ __device__ __forceinline__ uint32_t query_row(const GridDev& G, const QueryBox& 
     return g2 + gz * gz <= q.r2;
   };
   first = ((uint32_t)i * (uint32_t)cpd + (uint32_t)j) * (uint32_t)cpd;  // celery.rs:317-325
+  if (cell_by_cell(G)) {
+    first += (uint32_t)k;
+    return in(k) ? 1u : 0u;
+  }
   // the box's k nearest the query's
   const int near = q.hz < q.k0 ? q.k0 : (q.hz > q.k1 ? q.k1 : q.hz);
   if (!in(near)) return 0;
