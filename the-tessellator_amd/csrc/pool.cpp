@@ -18,8 +18,9 @@
 //
 // Bounded: at most 1/64 of the device's memory is kept, oldest blocks given
 // back first; a block is handed out for requests of at least 8/9 of it; all
-// of it is given back when an allocation fails and when the last context on
-// the device is destroyed.
+// of it is given back when a device allocation of any size finds no memory
+// (and that is tried once more), and when the last context on the device is
+// destroyed.
 #include <hip/hip_runtime.h>
 
 #include <list>
@@ -65,7 +66,25 @@ void give_back_all(DevicePool& P) {
   for (const KeptBlock& b : out) (void)hipFree(b.p);
 }
 
+DevicePool* current_pool(int* device) {
+  if (hipGetDevice(device) != hipSuccess) *device = -1;
+  return pool_of(*device);
+}
+
 }  // namespace
+
+hipError_t device_alloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  int device = -1;
+  DevicePool* P = e == hipErrorOutOfMemory ? current_pool(&device) : nullptr;
+  if (P) {
+    (void)hipGetLastError();
+    give_back_all(*P);
+    e = hipMalloc(p, bytes);
+  }
+  if (e != hipSuccess) *p = nullptr;
+  return e;
+}
 
 void pool_context_add(int device) {
   DevicePool* P = pool_of(device);
@@ -90,13 +109,9 @@ void pool_context_remove(int device) {
 hipError_t pool_alloc(size_t bytes, PoolBlock* out) {
   *out = PoolBlock{};
   int device = -1;
-  if (hipGetDevice(&device) != hipSuccess) device = -1;
-  hipError_t e = hipMalloc(&out->token, kTokenBytes);
-  if (e != hipSuccess) {
-    out->token = nullptr;
-    return e;
-  }
-  DevicePool* P = pool_of(device);
+  DevicePool* P = current_pool(&device);
+  hipError_t e = device_alloc(&out->token, kTokenBytes);
+  if (e != hipSuccess) return e;
   if (P) {
     std::lock_guard<std::mutex> g(P->mu);
     auto best = P->kept.end();
@@ -112,12 +127,7 @@ hipError_t pool_alloc(size_t bytes, PoolBlock* out) {
     }
   }
   if (!out->p) {
-    e = hipMalloc(&out->p, bytes);
-    if (e == hipErrorOutOfMemory && P) {
-      (void)hipGetLastError();
-      give_back_all(*P);
-      e = hipMalloc(&out->p, bytes);
-    }
+    e = device_alloc(&out->p, bytes);
     if (e != hipSuccess) {
       (void)hipFree(out->token);
       *out = PoolBlock{};

@@ -27,6 +27,9 @@ struct PoolBlock {
   int device = -1;
 };
 constexpr size_t kPoolMin = size_t(2) << 20;  // smaller ones the runtime suballocates
+// hipMalloc, tried again without the kept blocks where memory is out; *p is
+// null when it fails.
+hipError_t device_alloc(void** p, size_t bytes);
 hipError_t pool_alloc(size_t bytes, PoolBlock* out);
 void pool_free(const PoolBlock& b);
 // contexts on a device: with the last one its kept blocks go
@@ -69,7 +72,7 @@ struct DevBuf {
       e = pool_alloc(sizeof(T) * count, &block);
       p = static_cast<T*>(block.p);
     } else {
-      e = hipMalloc((void**)&p, sizeof(T) * count);
+      e = device_alloc((void**)&p, sizeof(T) * count);
     }
     if (e == hipSuccess) n = count;
     return e;
