@@ -238,6 +238,7 @@ tess_status prepare_tables(tess_batch* b, double* table_ms) {
     std::vector<TableBuild> tb(b->nsets);
     std::vector<size_t> at(b->nsets);
     std::vector<size_t> host;  // sets whose table the device does not build
+    TableBuild longest{};
     for (size_t s = 0; s < b->nsets; ++s) {
       const GridDev& G = b->hgrid[s];
       TableBuild& t = tb[s];
@@ -247,6 +248,7 @@ tess_status prepare_tables(tess_batch* b, double* table_ms) {
       t.sz = G.sz;
       t.L = (int)std::min<int64_t>(kTableL, (int64_t)G.cpd - 1);
       t.kcut = table_kcut(G.cpd, G.sx, G.sy, G.sz, t.L);
+      longest.L = std::max(longest.L, t.L);
       t.len = 0;
       at[s] = total;
       if (table_on_device(G.cpd, G.sx, G.sy, G.sz, t.L)) {
@@ -267,7 +269,7 @@ tess_status prepare_tables(tess_batch* b, double* table_ms) {
     tess_status st;
     if ((st = c->hip(hipMemcpy(b->tbuild.p, tb.data(), sizeof(TableBuild) * b->nsets, hipMemcpyHostToDevice),
                      "upload")) != TESS_OK ||
-        (st = c->hip(launch_table(b->tbuild.p, (int)b->nsets, TableBuild{}, c->stream), "shell tables")) != TESS_OK)
+        (st = c->hip(launch_table(b->tbuild.p, (int)b->nsets, longest, c->stream), "shell tables")) != TESS_OK)
       return st;
     for (size_t s : host) {
       TableBuild& t = tb[s];

@@ -134,7 +134,8 @@ hipError_t launch_pick_u64(const uint64_t* src, const uint64_t* at, int n, uint6
 
 // table.hip: the first len entries of the shell table of a grid shape (cpd
 // cells per dimension of sizes s), |o|_inf <= L, keys below kcut: as
-// build_table_host leaves them.  many: `count` of them (device), else `one`.
+// build_table_host leaves them.  many: `count` of them (device), one.L the
+// largest of their L; else `one`.
 constexpr int kTableDeviceL = 12;
 struct TableBuild {
   int64_t cpd;

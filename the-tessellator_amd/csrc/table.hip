@@ -84,11 +84,25 @@ __global__ __launch_bounds__(256) void k_table(const TableBuild* __restrict__ ma
 
 }  // namespace
 
+// Sets of a batch in grid y, whose documented limit is 65,536 on this device:
+// batches of more sets take several launches.
+constexpr int kTableSets = 32768;
+
 hipError_t launch_table(const TableBuild* many, int count, const TableBuild& one, hipStream_t s) {
-  const int w = 2 * (many ? kTableDeviceL : one.L) + 1;
-  hipLaunchKernelGGL(k_table, dim3((unsigned)((w * w * w * kTableLanes + 255) / 256), (unsigned)(many ? count : 1)), dim3(256), 0, s,
-                     many, one);
-  return hipGetLastError();
+  const int w = 2 * one.L + 1;
+  const dim3 block(256);
+  const unsigned x = (unsigned)((w * w * w * kTableLanes + 255) / 256);
+  if (!many) {
+    hipLaunchKernelGGL(k_table, dim3(x, 1), block, 0, s, many, one);
+    return hipGetLastError();
+  }
+  for (int at = 0; at < count; at += kTableSets) {
+    const int n = count - at < kTableSets ? count - at : kTableSets;
+    hipLaunchKernelGGL(k_table, dim3(x, (unsigned)n), block, 0, s, many + at, one);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 }  // namespace tess
