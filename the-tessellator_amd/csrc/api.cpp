@@ -621,12 +621,7 @@ tess_status tess_ctx_create(int dev, tess_ctx** out) {
   if (!c) return TESS_E_NOMEM;
   c->device = dev;
   (void)noalloc_setup(dev);  // the scratch address of this device, once
-  if (hipStreamCreate(&c->stream) != hipSuccess ||
-      hipHostMalloc((void**)&c->mail, sizeof(PassReport), hipHostMallocCoherent) != hipSuccess ||
-      hipHostMalloc(&c->up, tess_ctx::kUpBytes, hipHostMallocCoherent) != hipSuccess ||
-      hipEventCreateWithFlags(&c->up_ev, hipEventDisableTiming) != hipSuccess) {
-    if (c->stream) (void)hipStreamDestroy(c->stream);
-    c->mail = nullptr;
+  if (hipStreamCreate(&c->stream) != hipSuccess) {
     delete c;
     return TESS_E_DEVICE;
   }
@@ -669,7 +664,7 @@ tess_status tess_diagram_create(tess_ctx* ctx, const double* xyz, size_t n, cons
   // the kernel that splits the coordinates, with nothing to wait for (an
   // upload and its wait are 17 to 21 us: a diagram of 1,000 points 191 -> 169
   // us, of 16,000 407 -> 386; more would keep the host copying instead)
-  const bool staged = 24 * n <= tess_ctx::kUpBytes;
+  const bool staged = 24 * n <= tess_ctx::kUpBytes && ctx->up_ready();
   if (staged) {
     if (ctx->up_busy) st = ctx->hip(hipEventSynchronize(ctx->up_ev), "upload");
     if (st == TESS_OK) {

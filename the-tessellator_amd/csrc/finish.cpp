@@ -60,6 +60,11 @@ tess_status read_items(tess_ctx* c, const uint32_t* dev, uint32_t n, std::vector
 }
 
 tess_status pass_report(tess_ctx* c, const ReportArgs& a, const char* what) {
+  if (!c->mail && hipHostMalloc((void**)&c->mail, sizeof(PassReport), hipHostMallocCoherent) != hipSuccess) {
+    c->mail = nullptr;
+    (void)hipGetLastError();
+    return c->fail(TESS_E_NOMEM, "pinned host allocation failed");
+  }
   const tess_status st = c->hip(launch_pass_report(a, c->mail, c->stream), what);
   return st != TESS_OK ? st : c->hip(hipStreamSynchronize(c->stream), what);
 }

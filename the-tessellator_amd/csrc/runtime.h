@@ -145,13 +145,23 @@ struct tess_ctx {
   DevBuf<uint32_t> fin_tab, fin_cap;
   DevBuf<uint64_t> fin_tab64, fin_cap64;
   Staging stage;  // downloads (tess::download)
-  PassReport* mail = nullptr;  // pinned; under mu
-  // Points of small sets on their way to the device: pinned, with the event
-  // after the kernel that reads them; under mu.
+  // Pinned, made when first needed (a context is also made while a stream of
+  // the process is being captured, where the runtime refuses allocations);
+  // under mu.
+  PassReport* mail = nullptr;
+  // Points of small sets on their way to the device, with the event after the
+  // kernel that reads them; under mu.
   static constexpr size_t kUpBytes = size_t(1) << 20;
   void* up = nullptr;
   hipEvent_t up_ev = nullptr;
   bool up_busy = false;
+  bool up_ready() {
+    if (!up && hipHostMalloc(&up, kUpBytes, hipHostMallocCoherent) != hipSuccess) up = nullptr;
+    if (up && !up_ev && hipEventCreateWithFlags(&up_ev, hipEventDisableTiming) != hipSuccess) up_ev = nullptr;
+    if (up && up_ev) return true;
+    (void)hipGetLastError();
+    return false;
+  }
   ~tess_ctx() {
     if (mail) (void)hipHostFree(mail);
     if (up) (void)hipHostFree(up);
