@@ -136,18 +136,20 @@ void host_copy(char* dst, const char* src, size_t len) {
 
 namespace {
 
-// Without pinned memory: plain copies.
-hipError_t download_plain(const Piece* pieces, int count) {
-  for (int k = 0; k < count; ++k) {
+// A copy an array, on the context's stream.
+hipError_t download_plain(tess_ctx* c, const Piece* pieces, int count) {
+  uint64_t first[kCopyOutPieces] = {};
+  hipError_t e = hipSuccess;
+  for (int k = 0; k < count && e == hipSuccess; ++k) {
     const Piece& p = pieces[k];
-    if (!p.dst || !p.bytes) continue;
-    hipError_t e = hipMemcpy(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost);
-    uint64_t m = 0;
-    if (e == hipSuccess && p.sub) e = hipMemcpy(&m, p.sub, 8, hipMemcpyDeviceToHost);
-    if (e != hipSuccess) return e;
-    if (p.sub)
-      for (size_t i = 0; i < p.bytes / 8; ++i) static_cast<uint64_t*>(p.dst)[i] -= m;
+    e = hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess && p.sub) e = hipMemcpyAsync(&first[k], p.sub, 8, hipMemcpyDeviceToHost, c->stream);
   }
+  const hipError_t w = hipStreamSynchronize(c->stream);  // nothing left in flight, also after an error
+  if (e != hipSuccess || w != hipSuccess) return e != hipSuccess ? e : w;
+  for (int k = 0; k < count; ++k)
+    if (pieces[k].sub)
+      for (size_t i = 0; i < pieces[k].bytes / 8; ++i) static_cast<uint64_t*>(pieces[k].dst)[i] -= first[k];
   return hipSuccess;
 }
 
@@ -156,23 +158,30 @@ hipError_t download_plain(const Piece* pieces, int count) {
 hipError_t download(tess_ctx* c, const Piece* pieces, int count) {
   CopyOut a;
   std::memset(&a, 0, sizeof(a));
-  char* out[kCopyOutPieces];
-  uint64_t total = 0;
+  Piece live[kCopyOutPieces];
+  uint64_t total = 0, largest = 0;
   for (int k = 0; k < count; ++k) {
     if (!pieces[k].dst || !pieces[k].bytes) continue;
     if (a.npieces == kCopyOutPieces) return hipErrorInvalidValue;
-    out[a.npieces] = static_cast<char*>(pieces[k].dst);
+    live[a.npieces] = pieces[k];
     a.piece[a.npieces++] = {pieces[k].src, pieces[k].sub, total, pieces[k].bytes};
     total += (pieces[k].bytes + 15) & ~size_t(15);
+    largest = std::max<uint64_t>(largest, pieces[k].bytes);
   }
   if (!total) return hipSuccess;
+  constexpr size_t kOne = size_t(1) << 20, kLargeArray = size_t(16) << 20;
   // one chunk up to 1 MiB, else four and more of 1 to 64 MiB: transfers and
   // host copies overlap
-  constexpr size_t kOne = size_t(1) << 20;
   const size_t chunk =
       total <= kOne ? total : std::min(Staging::kBytes, std::max(kOne, (total / 4 + 4095) & ~size_t(4095)));
   Staging& S = c->stage;
-  std::lock_guard<std::mutex> g(S.mu);
+  // a download of small arrays does not wait for another one's turn with the
+  // buffers, which may be hundreds of MiB long
+  std::unique_lock<std::mutex> g(S.mu, std::defer_lock);
+  if (largest >= kLargeArray)
+    g.lock();
+  else if (!g.try_lock())
+    return download_plain(c, live, a.npieces);
   for (int k = 0; k < (total > chunk ? 2 : 1); ++k) {
     if (S.cap[k] < chunk) {
       if (S.buf[k]) (void)hipHostFree(S.buf[k]);
@@ -181,14 +190,16 @@ hipError_t download(tess_ctx* c, const Piece* pieces, int count) {
       S.cap[k] = 0;
       if (hipHostMalloc(&S.buf[k], cap, hipHostMallocCoherent) != hipSuccess) {
         S.buf[k] = nullptr;
-        return download_plain(pieces, count);
+        (void)hipGetLastError();
+        return download_plain(c, live, a.npieces);
       }
       S.cap[k] = cap;
     }
     if (!S.ev[k]) {
       if (hipEventCreateWithFlags(&S.ev[k], hipEventDisableTiming) != hipSuccess) {
         S.ev[k] = nullptr;
-        return download_plain(pieces, count);
+        (void)hipGetLastError();
+        return download_plain(c, live, a.npieces);
       }
     }
   }
@@ -210,7 +221,9 @@ hipError_t download(tess_ctx* c, const Piece* pieces, int count) {
     for (int k = 0; k < a.npieces; ++k) {
       const CopyOutPiece& p = a.piece[k];
       const uint64_t f = std::max(lo, p.start), t = std::min(hi, p.start + p.bytes);
-      if (f < t) host_copy(out[k] + (f - p.start), static_cast<const char*>(S.buf[i & 1]) + (f - lo), t - f);
+      if (f < t)
+        host_copy(static_cast<char*>(live[k].dst) + (f - p.start), static_cast<const char*>(S.buf[i & 1]) + (f - lo),
+                  t - f);
     }
   }
   if (e != hipSuccess) (void)hipStreamSynchronize(c->stream);  // nothing left in flight into the staging
