@@ -9,10 +9,11 @@
 // cells of a row (i, j) that the radius reaches are one interval of k (the
 // gap distance only grows away from the query's cell), and consecutive cells
 // are consecutive in the grid order, so a row is one run of points (or cell
-// ids) found from two delimiters.  Both passes give a query 16 lanes, a row
-// each; long rows are walked by the whole wavefront.  The neighbour cloud walks the shell
-// table in canonical order, 64 entries per step, until the first key above
-// the radius.
+// ids) found from two delimiters.  A query has 16 lanes, a row each, and long
+// rows are walked by the whole wavefront; the fill pass of a few thousand
+// queries and fewer gives each a wavefront.  The neighbour cloud walks the
+// shell table in canonical order, 64 entries per step, until the first key
+// above the radius.
 //
 // The points of a step's runs are walked one per lane, so loads and stores of
 // neighbouring lanes are neighbouring addresses.  Large query sets are taken
@@ -408,6 +409,40 @@ __global__ __launch_bounds__(256) void k_query_box(QueryArgs a) {
   if (live && sub == 0 && a.count) a.count[qi] = cursor;
 }
 
+// The same by a wavefront per query, 64 rows a step, for query sets too small
+// to fill the chip with four queries a wavefront, whose long rows are walked
+// one after the other for all four (kBoxWaveMax).
+template <int KIND, bool FILL>
+__global__ __launch_bounds__(256) void k_query_box_wave(QueryArgs a) {
+  constexpr int MODE = KIND == 0 ? 3 : (KIND == 1 ? 0 : 1);
+  __shared__ uint8_t heads[4][64];
+  uint8_t* head = heads[threadIdx.x >> 6];
+  const int lane = threadIdx.x & 63;
+  const uint32_t w = blockIdx.x * 4u + (threadIdx.x >> 6);
+  if (w >= (uint32_t)a.nq) return;
+  const uint32_t qi = a.order ? a.order[w] : w;
+  const double qx = a.q[3 * (size_t)qi], qy = a.q[3 * (size_t)qi + 1], qz = a.q[3 * (size_t)qi + 2];
+  const QueryBox q = query_box(a.g, qx, qy, qz, a.radius[(size_t)qi * a.rstride]);
+  uint64_t cursor = FILL ? a.offsets[qi] : 0;
+  const uint64_t begin = cursor, end = FILL ? a.offsets[qi + 1] : 0;
+  for (uint32_t base = 0; base < q.rows; base += 64) {
+    uint32_t s0 = 0, len = 0;
+    if ((uint32_t)lane < q.rows - base) {
+      uint32_t first;
+      const uint32_t n = query_row(a.g, q, base + (uint32_t)lane, first);
+      if (KIND == 0) {
+        s0 = first;
+        len = n;
+      } else if (n) {
+        s0 = a.delim[first];
+        len = a.delim[first + n] - s0;
+      }
+    }
+    emit_points<MODE, FILL>(a, s0, len, lane, qx, qy, qz, q.r2, cursor, end, head);
+  }
+  if (lane == 0 && a.count) a.count[qi] = (uint32_t)(cursor - begin);
+}
+
 // Cell::compute_neighbor_cloud: expand_all_in_radius from the query's grid
 // cell (celery.rs:1023-1075) + the group filter (interface.rs:358-361).  The
 // table covers every key <= the largest radius (or is the full order).
@@ -497,6 +532,22 @@ __global__ __launch_bounds__(256) void k_query_cloud_count(QueryArgs a) {
   if (live && sub == 15) a.count[qi] = (uint32_t)v;
 }
 
+// Queries up to which a box fill gets a wavefront each.  Real-radius calls over
+// 200k points, four queries a wavefront and one: 64 queries with 26,000 points
+// in their boxes 1,062 and 280 us, 4,096 of them 1,019 and 405, 8,192 1,089
+// and 543, 16,384 1,363 and 780; with 6 points in their boxes 72 and 69, 105
+// and 111, 104 and 113, 119 and 126, and falling behind from there (65,536:
+// 140 and 158).
+constexpr int kBoxWaveMax = 8192;
+
+template <int KIND, bool FILL>
+void launch_box(const QueryArgs& a, hipStream_t s) {
+  if (a.nq <= kBoxWaveMax)
+    hipLaunchKernelGGL((k_query_box_wave<KIND, FILL>), dim3((unsigned)((a.nq + 3) / 4)), dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((k_query_box<KIND, FILL>), dim3((unsigned)((a.nq + 15) / 16)), dim3(256), 0, s, a);
+}
+
 template <bool FILL>
 hipError_t launch_query_pass(const QueryArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)((a.nq + 3) / 4)), block(256);
@@ -504,18 +555,18 @@ hipError_t launch_query_pass(const QueryArgs& a, hipStream_t s) {
   switch (a.kind) {
     case 0:
       if (FILL)
-        hipLaunchKernelGGL((k_query_box<0, true>), grid16, block, 0, s, a);
+        launch_box<0, true>(a, s);
       else
         hipLaunchKernelGGL((k_query_box_count<0>), grid16, block, 0, s, a);
       break;
     case 1:
       if (FILL)
-        hipLaunchKernelGGL((k_query_box<1, true>), grid16, block, 0, s, a);
+        launch_box<1, true>(a, s);
       else
         hipLaunchKernelGGL((k_query_box_count<1>), grid16, block, 0, s, a);
       break;
     case 2:
-      hipLaunchKernelGGL((k_query_box<2, FILL>), grid16, block, 0, s, a);
+      launch_box<2, FILL>(a, s);
       break;
     default:
       if (!FILL && !a.groups && a.nq >= kCloudCountMin)
