@@ -738,11 +738,17 @@ hipError_t launch_bounds(const double* x, const double* y, const double* z, int 
 // The whole binning of a small set by one workgroup: bounds, grid, cell
 // counts, delimiters, points in grid order (ascending index in a cell), all
 // between the passes in LDS and registers.  A cell's points land in its range
-// by atomics, in no set order; each then counts the lower indices beside it.
-// Bound by the latency of its seven steps, above a few thousand points by what
-// one CU loads and stores.  It takes the place of ten launches, 55 us at any
-// of these sizes: 26 us at 1,000 points, 48 at 8,000, 60 at 12,000, where a
-// diagram still gains (355 -> 347 us; at 14,000 neither way is ahead).
+// by atomics, in no set order; each then counts the lower indices beside it,
+// or, in a cell of more than kBinDense points, takes its turn in index order.
+// Bound by the latency of its steps, above a few thousand points by what one
+// CU loads and stores.  Against ten launches, spread-out points: 27 us (80) at
+// 1,000 points, 43 (81) at 6,000, 61 (81) at 12,000, where a diagram still
+// gains (355 -> 347 us; at 14,000 neither way is ahead).  In clusters the ten
+// launches take longer, 12,000 points in ten clusters 208 us, here 125 (739
+// with every point of a cell looking at every other one), in one place 88.
+// Lines at 32, 64 and 128 points: 288, 263, 275 us for 12,000 points in 30
+// clusters (a call that bins), but 306, 276, 192 spread out at 100 a cell.
+constexpr uint32_t kBinDense = 128;
 template <int PER>
 __global__ __launch_bounds__(1024) void k_bin_small(const double* __restrict__ x, const double* __restrict__ y,
                                                     const double* __restrict__ z, int n, int cpd, int nbins,
@@ -750,11 +756,13 @@ __global__ __launch_bounds__(1024) void k_bin_small(const double* __restrict__ x
                                                     uint32_t* __restrict__ delim, uint32_t* __restrict__ sorted,
                                                     PointRec* __restrict__ pts) {
   __shared__ alignas(16) uint32_t cnt[kBinSmallCells + 4];
-  __shared__ uint16_t list[1024 * PER];
+  __shared__ alignas(16) uint16_t list[1024 * PER];
   __shared__ double red[6][16];
   __shared__ uint32_t wsum[2][16];
+  __shared__ uint32_t dense;  // whether a cell has more than kBinDense points
   const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
   double lo[3] = {x[0], y[0], z[0]}, hi[3] = {x[0], y[0], z[0]};
+  if (t == 0) dense = 0;
   for (int b = t; b < nbins; b += 1024) cnt[b] = 0;
 #pragma unroll 4
   for (int i = t; i < n; i += 1024) {
@@ -834,6 +842,7 @@ __global__ __launch_bounds__(1024) void k_bin_small(const double* __restrict__ x
       if (k0 + k < nbins) {
         cnt[k0 + k] = run;
         delim[k0 + k] = run;
+        if (v[k] > kBinDense) dense = 1;
       }
       run += v[k];
     }
@@ -854,12 +863,60 @@ __global__ __launch_bounds__(1024) void k_bin_small(const double* __restrict__ x
     const int i = t + 1024 * u;
     if (i < n) {
       const uint32_t s = cnt[b[u]], e = cnt[b[u] + 1];
+      if (e - s > kBinDense) continue;
       uint32_t k = s;
-      for (uint32_t q = s; q < e; ++q) k += list[q] < i ? 1u : 0u;
+      uint32_t q = s;
+      for (; q < e && (q & 7u); ++q) k += list[q] < i ? 1u : 0u;
+      for (; q + 8 <= e; q += 8) {  // eight ids a read
+        const uint4 w = *reinterpret_cast<const uint4*>(&list[q]);
+        const uint32_t two[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+        for (int h = 0; h < 4; ++h)
+          k += ((two[h] & 0xffffu) < (uint32_t)i ? 1u : 0u) + ((two[h] >> 16) < (uint32_t)i ? 1u : 0u);
+      }
+      for (; q < e; ++q) k += list[q] < i ? 1u : 0u;
       sorted[k] = (uint32_t)i;
       pts[k] = PointRec{x[i], y[i], z[i], (uint32_t)i, 0u};
     }
   }
+  if (!dense) return;
+  // dense cells: the points of the wavefront's 64 that share a cell, first of
+  // them in the low 6 bits, place among them in the next 6, their number from
+  // bit 12 on (0: not in a dense cell)
+  uint32_t same[PER];
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    same[u] = 0;
+    const bool in = t + 1024 * u < n && cnt[b[u] + 1] - cnt[b[u]] > kBinDense;
+    for (uint64_t left = __ballot(in); left;) {
+      const int first = __builtin_ctzll(left);
+      const int c = __builtin_amdgcn_readlane(b[u], first);
+      const uint64_t m = __ballot(in && b[u] == c);
+      if (m >> lane & 1)
+        same[u] = (uint32_t)first | (uint32_t)__popcll(m & ((1ull << lane) - 1ull)) << 6 | (uint32_t)__popcll(m) << 12;
+      left &= ~m;
+    }
+  }
+  // in index order, wavefront after wavefront: a dense cell's delimiter moves
+  // past the points that have their places (nothing else reads it any more)
+#pragma unroll
+  for (int u = 0; u < PER; ++u)
+    for (int w = 0; w < 16 && 1024 * u + 64 * w < n; ++w) {
+      __syncthreads();
+      if (w != wid || !__ballot(same[u] != 0)) continue;
+      const int first = (int)(same[u] & 63u);
+      uint32_t k = 0;
+      if (same[u] && first == lane) {
+        k = cnt[b[u]];
+        cnt[b[u]] = k + (same[u] >> 12);
+      }
+      k = __shfl(k, first, 64) + (same[u] >> 6 & 63u);
+      if (same[u]) {
+        const int i = t + 1024 * u;
+        sorted[k] = (uint32_t)i;
+        pts[k] = PointRec{x[i], y[i], z[i], (uint32_t)i, 0u};
+      }
+    }
 }
 
 namespace {
