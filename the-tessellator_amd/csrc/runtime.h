@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstring>
 #include <functional>
@@ -11,6 +12,7 @@
 #include <mutex>
 #include <string>
 #include <tuple>
+#include <utility>
 #include <vector>
 
 #include "launch.h"
@@ -85,6 +87,8 @@ struct Table {
   int len = 0;
   double kcut = 0;
   int L = 0;
+  uint64_t used = 0;  // the context's count of table calls at its last one
+  size_t bytes() const { return sizeof(double) * key.n + sizeof(int32_t) * off.n; }
 };
 
 // Shell table of a grid shape: entries with |o|_inf <= L in canonical order
@@ -133,8 +137,14 @@ struct tess_ctx {
   hipStream_t stream = nullptr;
   std::string err;
   std::mutex mu;
-  // shell tables keyed by (cpd, sx, sy, sz, L)
+  // Shell tables keyed by (cpd, sx, sy, sz, L).  A program whose points move
+  // has a new grid shape, and table, every step: past kTableBytes the least
+  // recently used go, down to half of it.  The last kTableKeep stay, so a
+  // call's own tables do (it doubles L up to six times).
   std::map<std::tuple<int64_t, uint64_t, uint64_t, uint64_t, int>, std::unique_ptr<Table>> tables;
+  static constexpr size_t kTableBytes = size_t(256) << 20, kTableKeep = 16;
+  size_t table_bytes = 0;
+  uint64_t table_calls = 0;
   DevBuf<double> diag;
   // spill kernel: workspaces (grown on demand), the pass's arguments, lists
   DevBuf<double> spill_d;
@@ -180,7 +190,10 @@ struct tess_ctx {
   Table* table(int64_t cpd, double sx, double sy, double sz, int L, tess_status* st) {
     auto key = std::make_tuple(cpd, bits(sx), bits(sy), bits(sz), L);
     auto it = tables.find(key);
-    if (it != tables.end()) return it->second.get();
+    if (it != tables.end()) {
+      it->second->used = ++table_calls;
+      return it->second.get();
+    }
     auto t = std::make_unique<Table>();
     if (table_on_device(cpd, sx, sy, sz, L)) {
       TableBuild b;
@@ -202,9 +215,7 @@ struct tess_ctx {
         *st = fail(TESS_E_DEVICE, "shell table failed");
         return nullptr;
       }
-      Table* r = t.get();
-      tables[key] = std::move(t);
-      return r;
+      return keep_table(key, std::move(t));
     }
     std::vector<double> k;
     std::vector<int32_t> o;
@@ -223,8 +234,25 @@ struct tess_ctx {
     t->len = (int)k.size();
     t->kcut = kc;
     t->L = L;
+    return keep_table(key, std::move(t));
+  }
+  Table* keep_table(const std::tuple<int64_t, uint64_t, uint64_t, uint64_t, int>& key, std::unique_ptr<Table> t) {
     Table* r = t.get();
+    r->used = ++table_calls;
+    table_bytes += r->bytes();
     tables[key] = std::move(t);
+    if (table_bytes <= kTableBytes || tables.size() <= kTableKeep) return r;
+    std::vector<std::pair<uint64_t, decltype(tables)::iterator>> all;  // newest first
+    for (auto e = tables.begin(); e != tables.end(); ++e) all.emplace_back(e->second->used, e);
+    std::sort(all.begin(), all.end(), [](const auto& x, const auto& y) { return x.first > y.first; });
+    size_t kept = 0, k = 0;
+    for (; k < all.size(); ++k) {
+      const size_t size = all[k].second->second->bytes();
+      if (k >= kTableKeep && kept + size > kTableBytes / 2) break;
+      kept += size;
+    }
+    for (; k < all.size(); ++k) tables.erase(all[k].second);
+    table_bytes = kept;
     return r;
   }
 };
