@@ -160,7 +160,10 @@ tess_status tess_ctx_synchronize(tess_ctx* ctx);
  * xyz: n points, AoS (x0,y0,z0,x1,...), copied for the call.  lo/hi: the
  * container box; every cell is the box clipped by bisectors (the reference's
  * container polyhedron, interface.rs:66-79).  The spatial grid is built over
- * the points' bounding box (celery.rs:81-125).  groups may be NULL. */
+ * the points' bounding box (celery.rs:81-125).  groups may be NULL.  xyz and
+ * groups are free again when the call returns; the upload of a set of up to
+ * 1 MiB without groups may then still be under way on the context's stream,
+ * which every later call on the diagram follows. */
 tess_status tess_diagram_create(tess_ctx* ctx, const double* xyz, size_t n, const double lo[3],
                                 const double hi[3], const int64_t* groups, const tess_opts* opts,
                                 tess_diagram** out);

@@ -706,9 +706,12 @@ tess_status tess_diagram_create(tess_ctx* ctx, const double* xyz, size_t n, cons
     if (st == TESS_OK) {
       std::memcpy(ctx->up, xyz, 24 * n);
       st = ctx->hip(launch_soa_host((const double*)ctx->up, (int)n, d->x.p, d->y.p, d->z.p, s), "upload");
+      ctx->up_busy = st == TESS_OK && hipEventRecord(ctx->up_ev, s) == hipSuccess;
+      if (st == TESS_OK && !ctx->up_busy) {  // no event for the next upload to wait for: the buffer is read now
+        (void)hipGetLastError();
+        st = ctx->hip(hipStreamSynchronize(s), "upload");
+      }
     }
-    if (st == TESS_OK) st = ctx->hip(hipEventRecord(ctx->up_ev, s), "upload");
-    ctx->up_busy = true;
   } else {
     if (d->xyz_tmp.alloc(3 * n) != hipSuccess) {
       delete d;
