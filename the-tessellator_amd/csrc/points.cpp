@@ -142,6 +142,7 @@ tess_status tess_diagram_cells_at_particles(tess_diagram* d, const double* xyz, 
   ra.tredo = T.tredo.p;
   ra.spill = T.spill.p;
   ra.total = p->foff.p + m;
+  ra.extra = (const uint64_t*)T.arena.p + (size_t)kArenaStride * (kArenaParts + 1);  // cells without room
   ra.summary = T.summary.p;
   auto offsets = [&]() -> tess_status {
     tess_status e = c->hip(hipEventRecord(ev.e[1], s), "event");
@@ -186,6 +187,7 @@ tess_status tess_diagram_cells_at_particles(tess_diagram* d, const double* xyz, 
   if ((nredo || ntab || nspill) && (st = offsets()) != TESS_OK) return st;
   p->total = c->mail->total;
   const Summary sm2 = c->mail->sum;
+  if (c->mail->extra) return c->fail(TESS_E_CAPACITY, "the face arena is full");
   if (p->nbr.alloc(p->total) != hipSuccess || p->area.alloc(p->total) != hipSuccess)
     return c->fail(TESS_E_NOMEM, "device allocation failed");
   float ms[2] = {0, 0};
