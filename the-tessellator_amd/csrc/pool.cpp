@@ -89,10 +89,9 @@ hipError_t device_alloc(void** p, size_t bytes) {
 void pool_context_add(int device) {
   DevicePool* P = pool_of(device);
   if (!P) return;
-  size_t total = 0;
-  if (hipDeviceTotalMem(&total, device) != hipSuccess) total = 0;
   std::lock_guard<std::mutex> g(P->mu);
-  P->limit = total / 64;
+  size_t total = 0;
+  if (!P->limit && hipDeviceTotalMem(&total, device) == hipSuccess) P->limit = total / 64;
   ++P->contexts;
 }
 
