@@ -204,8 +204,11 @@ struct QueryBox {
 // A z extent past the largest double has cells of infinite size: a gap of 0
 // cells is then no number (0 x inf) and out of reach, a gap of 1 and more in
 // reach of an infinite radius^2, and a row's cells in reach are no interval.
-// Its rows are taken cell by cell.
-__device__ __forceinline__ bool cell_by_cell(const GridDev& G) { return !(G.sz < (double)INFINITY); }
+// Its rows are taken cell by cell.  (Infinite or no number, by the exponent:
+// on the scalar unit.)
+__device__ __forceinline__ bool cell_by_cell(const GridDev& G) {
+  return ((uint32_t)((unsigned long long)__double_as_longlong(G.sz) >> 52) & 0x7ffu) == 0x7ffu;
+}
 
 __device__ __forceinline__ QueryBox query_box(const GridDev& G, double qx, double qy, double qz, double r) {
   QueryBox q;
@@ -237,10 +240,10 @@ __device__ __forceinline__ QueryBox query_box(const GridDev& G, double qx, doubl
 // bounded on the other side by the box.
 __device__ __forceinline__ uint32_t query_row(const GridDev& G, const QueryBox& q, uint32_t t, uint32_t& first) {
   const int cpd = G.cpd;
-  int k = 0;
+  int ka = q.k0, kb = q.k1;
   if (cell_by_cell(G)) {
     const uint32_t nk = (uint32_t)(q.k1 - q.k0 + 1);
-    k = q.k0 + (int)(t % nk);
+    ka = kb = q.k0 + (int)(t % nk);
     t /= nk;
   }
   const int i = q.i0 + (int)(t / q.nj), j = q.j0 + (int)(t % q.nj);
@@ -251,14 +254,9 @@ __device__ __forceinline__ uint32_t query_row(const GridDev& G, const QueryBox& 
     return g2 + gz * gz <= q.r2;
   };
   first = ((uint32_t)i * (uint32_t)cpd + (uint32_t)j) * (uint32_t)cpd;  // celery.rs:317-325
-  if (cell_by_cell(G)) {
-    first += (uint32_t)k;
-    return in(k) ? 1u : 0u;
-  }
   // the box's k nearest the query's
-  const int near = q.hz < q.k0 ? q.k0 : (q.hz > q.k1 ? q.k1 : q.hz);
+  const int near = q.hz < ka ? ka : (q.hz > kb ? kb : q.hz);
   if (!in(near)) return 0;
-  int ka = q.k0, kb = q.k1;
   for (int hi = near; ka < hi;) {  // the smallest k in reach is in ka .. hi
     const int mid = (ka + hi) >> 1;
     if (in(mid))
