@@ -7,8 +7,8 @@
 //
 //   graph 1 (captured once): binning of every set + a check that every point
 //            was binned
-//   host:    grid download, shell tables (built in parallel, cached by grid
-//            shape), per-set kernel arguments
+//   host:    grid download; shell tables of all sets built in one launch when
+//            a grid has changed; per-set kernel arguments
 //   plan:    item list in set order, or the learned order (features +
 //            inference + cost sort over all sets)
 //   graph 2 (captured per schedule shape, then replayed): the first pass over
@@ -28,7 +28,6 @@
 #include <map>
 #include <new>
 #include <sstream>
-#include <thread>
 #include <vector>
 
 #include "runtime.h"

@@ -544,7 +544,6 @@ __global__ __launch_bounds__(256) void k_grad_sum(const float* __restrict__ grad
   if (i < kMlpParams && threadIdx.x < 64) out[i] = g;
 }
 
-// Standardise targets: Tn = (T - mean) / std per column.
 // Per column the sum of T, or of (T - mean)^2 when the blocks' sums are given:
 // 256 blocks, each thread a strided row sum, then a tree.  Bound by latency:
 // 400k rows 16 us for both and the end, 720 us on a host thread with the
@@ -587,6 +586,7 @@ __global__ __launch_bounds__(256) void k_moments_end(double* __restrict__ part) 
     for (int k = 0; k < 4; ++k) part[k] = r[k];
 }
 
+// Standardise targets: Tn = (T - mean) / std per column.
 __global__ void k_standardise(const float* __restrict__ T, size_t n, float m0, float s0, float m1, float s1,
                               float* __restrict__ Tn) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;

@@ -60,6 +60,7 @@ struct NaArena {
   GridDev grid;
   Summary summary;
   CellArgs args;
+  // (fields that are gone: the header states the array's size)
   unsigned char reserved[40 + 4 * kNaBins];
   int32_t toff[kNaTable];
   int32_t snbr[kNaPoints * kNaFaces];

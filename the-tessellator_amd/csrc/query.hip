@@ -93,9 +93,10 @@ __device__ __forceinline__ uint32_t wave_excl(uint32_t v, int lane, uint32_t* to
 }
 
 // Runs of at least this many points (on average over a step's runs) are
-// walked one by one by the whole wavefront: no search for a position's run,
-// but the last 64 of every run are part empty.  At 1M clustered points (290 a
-// run) the fill pass of 1M real-radius queries took 1.92 ms so and 2.45 ms
+// walked one by one by the whole wavefront: no search for a position's run
+// (or, with 16 lanes a query, four times the lanes), but the last 64 of every
+// run are part empty.  At 1M clustered points (290 a run) the fill pass of 1M
+// real-radius queries took 1.92 ms with a wavefront per query so and 2.45 ms
 // with the runs' concatenation searched; between 15 and 35 points a run the
 // two forms are within 5 %.
 constexpr uint32_t kRunWalkMin = 48;
