@@ -186,7 +186,9 @@ tess_status tess_diagram_total_faces(const tess_diagram* d, uint64_t* out);
  * The arrays of a call (here and in the other *_copy* calls) come down
  * together through two pinned host buffers of 1 to 64 MiB that the context
  * allocates when they are needed and keeps until tess_ctx_destroy, copied out
- * by up to eight host threads; calls on one context take the buffers in turn. */
+ * by up to eight host threads; calls on one context take the buffers in turn,
+ * arrays below 16 MiB not waiting for their turn but copied one by one.
+ * Destinations in pinned memory are copied to directly. */
 tess_status tess_diagram_copy_cells(const tess_diagram* d, double* volume, uint32_t* face_count,
                                     uint64_t* face_offset, int32_t* neighbor, double* face_area);
 tess_status tess_diagram_device_cells(const tess_diagram* d, tess_cells_device* out);

@@ -822,10 +822,11 @@ __device__ __forceinline__ uint64_t mask_at(uint64_t reversed, uint32_t t) {
 // 4.33 -> 4.0, with the checks for room as one.
 // Measured with the rest of the cut path rewritten to the same ends (scalar
 // bookkeeping per cut instead of per test, arguments reloaded instead of
-// spilled): 20.7k instructions per uniform cell instead of 27.9k, no spilled
-// vector registers; cell pass of 1M uniform points 23.4 -> 18.3 ms, of 2M
+// spilled): 20.7k instructions per uniform cell instead of 27.9k (15.8k now,
+// with the two forms and the pre-test's order), no spilled vector registers; cell pass of 1M uniform points 23.4 -> 18.3 ms, of 2M
 // clustered 73.5 -> 58.7 ms, of a 256k FCC lattice 5.8 -> 4.6 ms.  Bound by
-// issue: VALU 75 % and scalar unit 69 % busy.
+// issue: VALU 75 % and scalar unit 63 % busy on uniform cells, 79 % and 59 %
+// on clustered ones.
 template <bool TWO, int PPL>
 __device__ __forceinline__ int clip_fast64(Lds<1, PPL, 1>& S, CellState<1, PPL, 1>& C, const uint64_t OM,
                                            const uint64_t INC, double pnx, double pny, double pnz, double off,
